@@ -40,9 +40,26 @@ constexpr int kQRows = 256;        // rows per workgroup (4 waves x 4 tiles of 1
 constexpr int kQHalf = 16;         // outputs j per workgroup
 constexpr int kQKL = kQR * kQR;    // contraction length
 
+// Where row m's operands start in ua and ub, in floats. Plain rows (w = 0): m ld_in in both. Rows of
+// the pair basis (w node pairs, nq basis rows per leaf, n leaves; see leaf_pair_level_kernel):
+// m = (ci nq + cj) w + p takes basis row ci of leaf 2p from ua and cj of leaf 2p + 1 from ub, both
+// [nq][n][ld_in].
+struct MergeRows {
+  int64_t ld_in;
+  int w, nq, n;
+  __device__ __forceinline__ void at(int64_t m, int64_t& a, int64_t& b) const {
+    a = b = m * ld_in;
+    if (w == 0) return;
+    const int c = static_cast<int>(m / w), p = static_cast<int>(m - static_cast<int64_t>(c) * w);
+    const int ci = c / nq, cj = c - ci * nq;
+    a = (static_cast<int64_t>(ci) * n + 2 * p) * ld_in;
+    b = (static_cast<int64_t>(cj) * n + 2 * p + 1) * ld_in;
+  }
+};
+
 __global__ void __launch_bounds__(256, 2)
 quadrilinear_merge_kernel(const float* __restrict__ T, const float* __restrict__ ua, const float* __restrict__ ub,
-                          float* __restrict__ out, int64_t M, int G, int64_t ld_in) {
+                          float* __restrict__ out, int64_t M, int G, MergeRows rows) {
   __shared__ float Ts[kQKL * kQHalf];  // Ts[kl][jj] = T[i][16 jh + jj][k][l], kl = 32 k + l
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -50,7 +67,7 @@ quadrilinear_merge_kernel(const float* __restrict__ T, const float* __restrict__
   const int i = blockIdx.y;
   const int jh = blockIdx.z;
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kQRows + wave * 64;
-  const int64_t ld = static_cast<int64_t>(G) * kQR;  // floats per row of out (ld_in: of a and b)
+  const int64_t ld = static_cast<int64_t>(G) * kQR;  // floats per row of out
 
   // stage T_i's half: thread t takes output jj = t mod 16 and 4 consecutive kl per pass
   const float* Ti = T + (static_cast<int64_t>(i) * kQR + kQHalf * jh) * kQKL;
@@ -70,8 +87,10 @@ quadrilinear_merge_kernel(const float* __restrict__ T, const float* __restrict__
   for (int rt = 0; rt < 4; ++rt) {
     const int64_t row = row0 + 16 * rt + c;
     const bool ok = row < M;
-    const float* ar = ua + (ok ? row : 0) * ld_in + i * kQR;
-    const float* br = ub + (ok ? row : 0) * ld_in + i * kQR;
+    int64_t ao, bo;
+    rows.at(ok ? row : 0, ao, bo);
+    const float* ar = ua + ao + i * kQR;
+    const float* br = ub + bo + i * kQR;
 #pragma unroll
     for (int q = 0; q < kQR / 4; ++q) {
       const float4 v = ok ? *reinterpret_cast<const float4*>(ar + 4 * q) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -615,6 +634,172 @@ __global__ void __launch_bounds__(256) readout_kernel(const float* __restrict__ 
   phase[b] = atan2f(im, re);
 }
 
+// --------------------------------------------------------------------------------------
+// The leaf and the first level through a basis of the walkers' inputs
+// --------------------------------------------------------------------------------------
+// Everything from a site's input q [nq] to the first merge is linear in q: the leaf carrier is
+// u = sum_c q_c E[c], E[c] = ((W_q[c] V) o h) U, and a node of the first level is bilinear,
+// out = sum_cd q_c q'_d O[c, d] with O the level's merge and residual apply of E[c] and E'[d].
+// So the leaf's and the first level's products run on nq rows per leaf and nq^2 rows per pair
+// instead of on every walker's rows, and this kernel forms each walker's carrier from them: the
+// leaf carriers' norms, the normalised coefficients, the node's sum, its rescale and its gate
+// (normalize_rows_kernel and level_gate_kernel of the plain path). At 1024 walkers of 64 sites
+// with nq = 4 the products fall from 65536 leaf and 32768 pair rows to 256 and 512.
+// A workgroup owns 16 walkers of one node pair p, its waves a quarter of the columns each.
+// Orientation: basis columns x walkers on
+// v_mfma_f32_16x16x4_f32, the contraction over c (leaf) or, in four steps, over (c, d); the row
+// of 16 columns a lane's register holds is one 16-byte store, 64 bytes per walker. Three passes
+// over the columns: leaf norms, the node's norm, the stores (the sums are formed again: the
+// basis is in L2 and the products are few). 107 us at 1024 x 64 sites, 41 of them for the 201 MB of
+// carriers it writes (139 us with a wave per 16 walkers and every column: too few waves).
+constexpr int kMaxBasis = 4;  // inputs per site the pair basis serves (one K step of the products)
+
+__global__ void __launch_bounds__(256) leaf_basis_kernel(const float* __restrict__ Wq, const float* __restrict__ V,
+                                                         const float* __restrict__ h, float* __restrict__ out, int n,
+                                                         int d_z, int R) {
+  // out[(c n + s) R + r] = (sum_z W_q[c, z] V[z, r]) h[s, r]
+  const int r = blockIdx.x * 256 + threadIdx.x;
+  if (r >= R) return;
+  const int c = blockIdx.y;
+  float a = 0.f;
+  for (int z = 0; z < d_z; ++z) a = fmaf(Wq[c * d_z + z], V[static_cast<int64_t>(z) * R + r], a);
+  for (int s = blockIdx.z; s < n; s += gridDim.z)
+    out[(static_cast<int64_t>(c) * n + s) * R + r] = a * h[static_cast<int64_t>(s) * R + r];
+}
+
+__global__ void __launch_bounds__(256) leaf_pair_level_kernel(const float* __restrict__ E, const float* __restrict__ O,
+                                                               const float* __restrict__ q,
+                                                               const uint8_t* __restrict__ opcodes,
+                                                               float* __restrict__ u_out, float* __restrict__ s_out,
+                                                               int64_t B, int n, int nq, int d, float eps) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane >> 4, c = lane & 15;
+  const int p = blockIdx.y, w = n / 2;
+  const int64_t b = static_cast<int64_t>(blockIdx.x) * 16 + c;
+  const bool ok = b < B;
+  // this wave's columns, in steps of 32 (d is a multiple of 32)
+  const int steps = d / 32;
+  const int t0 = 32 * (steps * wave / 4), t1 = 32 * (steps * (wave + 1) / 4);
+  __shared__ float part[3][4][16];  // per wave and walker: sums of squares (left leaf, right leaf, node)
+  float ql[kMaxBasis], qr[kMaxBasis];
+#pragma unroll
+  for (int s = 0; s < kMaxBasis; ++s) {
+    const float* qb = q + ((ok ? b : 0) * n + 2 * p) * nq;
+    ql[s] = s < nq ? qb[s] : 0.f;
+    qr[s] = s < nq ? qb[nq + s] : 0.f;
+  }
+  // this lane group's basis row; past nq (coefficient 0) any row
+  const int gr = g < nq ? g : 0;
+  const float* El = E + (static_cast<int64_t>(gr) * n + 2 * p) * d + c;
+  const float* Er = El + d;
+  const float* Os[kMaxBasis];
+#pragma unroll
+  for (int s = 0; s < kMaxBasis; ++s) Os[s] = O + (static_cast<int64_t>((s < nq ? s : 0) * nq + gr) * w + p) * d + c;
+  auto lane_of = [&](const float (&x)[kMaxBasis]) { return g == 0 ? x[0] : (g == 1 ? x[1] : (g == 2 ? x[2] : x[3])); };
+
+  // leaf carriers' norms: rms = sqrt(mean(u^2) + 1e-30)
+  float bl = lane_of(ql), br = lane_of(qr);
+  float ssl = 0.f, ssr = 0.f;
+  for (int t = t0; t < t1; t += 32) {
+    float al[2], ar[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      al[j] = El[t + 16 * j];
+      ar[j] = Er[t + 16 * j];
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const v4f ul = mfma16x4(al[j], bl, zero4()), ur = mfma16x4(ar[j], br, zero4());
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        ssl = fmaf(ul[r], ul[r], ssl);
+        ssr = fmaf(ur[r], ur[r], ssr);
+      }
+    }
+  }
+  ssl = group_sum(ssl);
+  ssr = group_sum(ssr);
+  if (g == 0) {
+    part[0][wave][c] = ssl;
+    part[1][wave][c] = ssr;
+  }
+  __syncthreads();
+  auto whole = [&](int i) { return (part[i][0][c] + part[i][1][c]) + (part[i][2][c] + part[i][3][c]); };
+  const float fd = static_cast<float>(d);
+  const float rl = sqrtf(whole(0) / fd + 1e-30f), rr = sqrtf(whole(1) / fd + 1e-30f);
+  bl /= rl;
+  br /= rr;
+  float co[kMaxBasis];
+#pragma unroll
+  for (int s = 0; s < kMaxBasis; ++s) co[s] = ql[s] / rl * br;
+  // the node's sum in columns t .. t + 31
+  auto node = [&](int t, v4f (&o)[2]) {
+    float a[2][kMaxBasis];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int s = 0; s < kMaxBasis; ++s) a[j][s] = Os[s][t + 16 * j];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      o[j] = zero4();
+#pragma unroll
+      for (int s = 0; s < kMaxBasis; ++s) o[j] = mfma16x4(a[j][s], co[s], o[j]);
+    }
+  };
+  float ss = 0.f;
+  for (int t = t0; t < t1; t += 32) {
+    v4f o[2];
+    node(t, o);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ss = fmaf(o[j][r], o[j][r], ss);
+  }
+  ss = group_sum(ss);
+  if (g == 0) part[2][wave][c] = ss;
+  __syncthreads();
+  const float scale = sqrtf(whole(2) / fd + eps);
+  const float inv = 1.0f / scale;
+  const int op = opcodes[p];
+  const float both = op == 0 ? 1.f : 0.f, left = op == 1 ? 1.f : 0.f, right = op == 2 ? 1.f : 0.f;
+  float* urow = u_out + ((ok ? b : 0) * w + p) * d + 4 * g;
+  for (int t = t0; t < t1; t += 32) {
+    v4f o[2];
+    node(t, o);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[j][r] *= inv;
+      if (op != 0) {
+        const v4f ul = mfma16x4(El[t + 16 * j], bl, zero4()), ur = mfma16x4(Er[t + 16 * j], br, zero4());
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[j][r] = both * o[j][r] + left * ul[r] + right * ur[r];
+      }
+      if (ok) *reinterpret_cast<v4f*>(urow + t + 16 * j) = o[j];
+    }
+  }
+  if (ok && g == 0 && wave == 0) {
+    const float sl = logf(rl), sr = logf(rr);
+    s_out[b * w + p] = both * (sl + sr + logf(scale)) + left * sl + right * sr;
+  }
+}
+
+// Whether the basis serves: at least one pair, inputs that fit its one K step, and no more basis
+// rows than walker rows, neither at the leaves (2 nq: the basis is held in half a leaf buffer) nor
+// at the pairs (nq^2). At that line (16 walkers, nq = 4, fine-tune widths) the whole wavefunction
+// takes 948 -> 732 us at 64 sites and 660 -> 456 us at 8; 500 x 64 sites 4618 -> 1978 us, 1024 x 64
+// 8799 -> 3386 us.
+bool basis_serves(int64_t B, int n, int nq) {
+  return n > 1 && nq <= kMaxBasis && B >= static_cast<int64_t>(nq) * nq && B >= 2 * nq;
+}
+
+hipError_t launch_merge(const float* T, const float* ua, const float* ub, float* out, int64_t M, int G,
+                        const MergeRows& rows, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>((M + kQRows - 1) / kQRows), static_cast<unsigned>(G), 2);
+  hipLaunchKernelGGL(quadrilinear_merge_kernel, grid, dim3(256), 0, stream, T, ua, ub, out, M, G, rows);
+  return hipGetLastError();
+}
+
 // Workspace sections of the whole-wavefunction executor, in floats, each rounded up to 64
 // floats (256 bytes).
 struct WaveFnWorkspace {
@@ -655,24 +840,49 @@ hipError_t launch_compiled_wavefunction(const WaveFnParams& p, hipStream_t strea
   const int64_t rows = p.B * p.n;
   const int G = p.d_m / kQR;
   hipError_t err;
-  // leaf: z = q W_q; u = ((z V) o leaf_h[site]) U; carriers RMS-normalised, s = log rms
-  if ((err = launch_gemm<kEpiPlain>(p.q, p.q_weight, z, nullptr, rows, p.d_z, p.d_q, 1, 0, stream)) != hipSuccess)
-    return err;
-  if ((err = apply_rows(z, p.leaf_V, p.leaf_h, p.leaf_U, nullptr, u_buf[0], work, rows, p.d_z, p.r_leaf, p.d_m, p.n, 0,
-                        stream, u_buf[1], u_cap[1])) != hipSuccess)
-    return err;
-  hipLaunchKernelGGL(normalize_rows_kernel, dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(256), 0, stream,
-                     u_buf[0], s_buf[0], rows, p.d_m);
-  if ((err = hipGetLastError()) != hipSuccess) return err;
+  int cur = 0, level = 0, width = p.n / 2;
+  if (basis_serves(p.B, p.n, p.d_q)) {
+    // E in the second carrier buffer, the first level's node basis in raw, carriers into the first
+    const int64_t er = static_cast<int64_t>(p.d_q) * p.n, pr = static_cast<int64_t>(p.d_q) * p.d_q * width;
+    hipLaunchKernelGGL(leaf_basis_kernel,
+                       dim3(static_cast<unsigned>((p.r_leaf + 255) / 256), static_cast<unsigned>(p.d_q),
+                            static_cast<unsigned>(p.n < 16 ? p.n : 16)),
+                       dim3(256), 0, stream, p.q_weight, p.leaf_V, p.leaf_h, work, p.n, p.d_z, p.r_leaf);
+    if ((err = hipGetLastError()) != hipSuccess) return err;
+    if ((err = launch_gemm<kEpiPlain>(work, p.leaf_U, u_buf[1], nullptr, er, p.d_m, p.r_leaf, 1, 0, stream, u_buf[0],
+                                      u_cap[0])) != hipSuccess)
+      return err;
+    if ((err = launch_merge(p.merge_T, u_buf[1], u_buf[1], raw, pr, G, MergeRows{p.d_m, width, p.d_q, p.n}, stream)) !=
+        hipSuccess)
+      return err;
+    if ((err = apply_rows(raw, p.merge_V, p.merge_h, p.merge_U, raw, raw, work, pr, p.d_m, p.r_merge, p.d_m, width, 0,
+                          stream, u_buf[0], u_cap[0])) != hipSuccess)
+      return err;
+    hipLaunchKernelGGL(leaf_pair_level_kernel,
+                       dim3(static_cast<unsigned>((p.B + 15) / 16), static_cast<unsigned>(width)), dim3(256), 0, stream,
+                       u_buf[1], raw, p.q, p.opcodes, u_buf[0], s_buf[0], p.B, p.n, p.d_q, p.d_m, p.merge_eps);
+    if ((err = hipGetLastError()) != hipSuccess) return err;
+    level = 1;
+    width /= 2;
+  } else {
+    // leaf: z = q W_q; u = ((z V) o leaf_h[site]) U; carriers RMS-normalised, s = log rms
+    if ((err = launch_gemm<kEpiPlain>(p.q, p.q_weight, z, nullptr, rows, p.d_z, p.d_q, 1, 0, stream)) != hipSuccess)
+      return err;
+    if ((err = apply_rows(z, p.leaf_V, p.leaf_h, p.leaf_U, nullptr, u_buf[0], work, rows, p.d_z, p.r_leaf, p.d_m, p.n,
+                          0, stream, u_buf[1], u_cap[1])) != hipSuccess)
+      return err;
+    hipLaunchKernelGGL(normalize_rows_kernel, dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(256), 0, stream,
+                       u_buf[0], s_buf[0], rows, p.d_m);
+    if ((err = hipGetLastError()) != hipSuccess) return err;
+  }
   // levels: node pairs (2p, 2p + 1) merged into node p, widths n/2, n/4, ..., 1
-  int cur = 0;
-  for (int level = 0, width = p.n / 2; width >= 1; ++level, width /= 2) {
+  for (; width >= 1; ++level, width /= 2) {
     const int64_t m = p.B * width;
     const float* u_in = u_buf[cur];
     const float* h_level = p.merge_h + static_cast<int64_t>(level) * (p.n / 2) * p.r_merge;
     const uint8_t* ops = p.opcodes + static_cast<int64_t>(level) * (p.n / 2);
-    if ((err = launch_quadrilinear_merge(p.merge_T, u_in, u_in + p.d_m, raw, m, G, 2 * static_cast<int64_t>(p.d_m),
-                                         stream)) != hipSuccess)
+    if ((err = launch_merge(p.merge_T, u_in, u_in + p.d_m, raw, m, G, MergeRows{2 * static_cast<int64_t>(p.d_m), 0, 1, 1},
+                            stream)) != hipSuccess)
       return err;
     // out = raw + ((raw V) o h_level[node]) U, written over raw
     if ((err = apply_rows(raw, p.merge_V, h_level, p.merge_U, raw, raw, work, m, p.d_m, p.r_merge, p.d_m, width, 0,
@@ -694,9 +904,7 @@ hipError_t launch_compiled_wavefunction(const WaveFnParams& p, hipStream_t strea
 
 hipError_t launch_quadrilinear_merge(const float* T, const float* ua, const float* ub, float* out, int64_t M, int G,
                                      int64_t ld_in, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>((M + kQRows - 1) / kQRows), static_cast<unsigned>(G), 2);
-  hipLaunchKernelGGL(quadrilinear_merge_kernel, grid, dim3(256), 0, stream, T, ua, ub, out, M, G, ld_in);
-  return hipGetLastError();
+  return launch_merge(T, ua, ub, out, M, G, MergeRows{ld_in, 0, 1, 1}, stream);
 }
 
 hipError_t launch_factorized_apply(const float* x, const float* V, const float* h, const float* U,

@@ -189,6 +189,36 @@ def test_compiled_wavefunction_matches_oracle(B, n, d_q, d_z, R_leaf, G, R_merge
     assert np.median(kappa) < 10  # most walkers are well conditioned: the bound is mostly the max-norm one
 
 
+@pytest.mark.parametrize(
+    "B,n,d_q,G,real",
+    [
+        (16, 2, 4, 2, "all"),      # the fewest walkers the pair basis serves (d_q^2), one pair
+        (15, 2, 4, 2, "all"),      # one fewer: the plain path
+        (9, 4, 3, 1, "random"),    # d_q below the basis width, 32 columns (three of four waves idle)
+        (4, 8, 2, 3, "sparse"),    # 96 columns, carries and empty nodes
+        (2, 4, 1, 2, "all"),
+        (17, 8, 4, 5, "sparse"),   # a second, nearly empty block of walkers
+        (70, 16, 5, 2, "random"),  # wider inputs: the plain path
+    ],
+)
+def test_compiled_wavefunction_pair_basis(B, n, d_q, G, real):
+    """The leaf and first level through the basis of the inputs (d_q <= 4, B >= max(d_q^2, 2 d_q)),
+    at its edges, with the bound of the test above."""
+    from hamiltonzero_amd import executor
+
+    _say(f"wavefunction basis B={B} n={n} d_q={d_q} G={G} {real}")
+    p = _wavefn_case(B * 5 + n + d_q, B, n, d_q, 20, 40, G, 36, 12, real)
+    kernel, tree, q = _namespaces(p)
+    la, ph = executor.execute_wavefunction(kernel, tree, q)
+    torch.cuda.synchronize()
+    want_la, want_ph = X.execute_wavefunction(**p)
+    kappa = _readout_condition(p)
+    dla = np.abs(la.cpu().numpy().astype(np.float64) - want_la)
+    assert np.all(dla <= TOL * np.max(np.abs(want_la)) + 1e-6 * kappa), (dla.max(), kappa[np.argmax(dla)])
+    dphi = np.abs(np.angle(np.exp(1j * (ph.cpu().numpy().astype(np.float64) - want_ph))))
+    assert np.all(dphi <= TOL * np.pi + 1e-6 * kappa), (dphi.max(), kappa[np.argmax(dphi)])
+
+
 def test_compiled_wavefunction_structure_errors():
     from hamiltonzero_amd import executor
 
