@@ -1,21 +1,21 @@
-// The compiled per-walker executor's products on the float32 matrix cores
-// (v_mfma_f32_16x16x4_f32): the quadrilinear merge of the tree levels and the factorized
-// apply ((x V) o h) U of the leaf, merge and readout factors.
+// The compiled per-walker executor's products: the quadrilinear merge of the tree levels and the
+// factorized apply ((x V) o h) U of the leaf, merge and readout factors, float32 throughout, their
+// products as sums of bfloat16 products (split_f32.h).
 //
 // Quadrilinear merge, out[m, iR + j] = sum_{k,l} T[i, j, k, l] a[m, iR + k] b[m, iR + l]:
-// for one group i it is one GEMM with a contraction of length R^2 = 1024,
-//     out_i[m, j] = sum_kl P_i[m, kl] T_i[kl, j],     P_i[m, kl] = a[m, iR + k] b[m, iR + l],
-// whose left operand P_i is never materialised: a lane holds its row's 32 values of a and 8
-// values of b and forms each operand value with one multiply right before its product.
-// A workgroup owns one group i, one half of the 32 outputs j and 256 rows; T_i's half
-// (1024 x 16 floats, 64 KiB) is staged in LDS once and read by every product step (one
-// 4-byte read feeds the four 16-row tiles of a wave). Two workgroups per compute unit.
+// for one group i and each k the inner sum is a product with a contraction of length R = 32,
+//     w_k[j, m] = sum_l T_i[j, k, l] b[m, iR + l],     out_i[m, j] = sum_k a[m, iR + k] w_k[j, m],
+// so b is split once and stays in registers, T_i streams through LDS in chunks of four k (48 KB
+// for two chunks), split as it is staged, and the outer sum is one multiply-add per element of
+// w_k in the matrix cores' output layout (16 vector instructions per 12 matrix ones). Bound by the
+// matrix cores' power: 73% busy at 1.66 GHz, 209 TFLOP/s of float32 products at 16384 rows, G = 48
+// (246 us; 514 with the contraction over (k, l) on the float32 matrix instruction).
 //
 // Factorized apply: two launches of one tiled GEMM, C = A B with A [M, K], B [K, N]
 // row-major; the first multiplies its result by the conditioner row of each output row
 // (h[m mod h_rows], one row per tree node, broadcast over walkers) before storing, the
-// second optionally adds a residual (the merge level's raw + apply(raw)). 128 x 128 output
-// tiles per 256-thread workgroup, 16-deep K slices double-buffered through LDS.
+// second optionally adds a residual (the merge level's raw + apply(raw)). 177 TFLOP/s at 65536 rows
+// of 1536 x 1024 x 1536 (123 with the float32 matrix instruction), 583 us at 16384 (866).
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -23,6 +23,7 @@
 
 #include "mhsea_device.h"
 #include "mhsea_launch.h"
+#include "split_f32.h"
 
 // Workspace of hz_factorized_apply_noalloc: kApplyScratchFloats floats (32 MiB) per device,
 // held from the library's first use on that device until the process ends. Every call on a
@@ -36,9 +37,7 @@ namespace {
 // Quadrilinear merge (R = 32)
 // --------------------------------------------------------------------------------------
 constexpr int kQR = 32;            // rank of the merge tensor
-constexpr int kQRows = 256;        // rows per workgroup (4 waves x 4 tiles of 16)
-constexpr int kQHalf = 16;         // outputs j per workgroup
-constexpr int kQKL = kQR * kQR;    // contraction length
+constexpr int kQK = 4;             // k per staged chunk of T_i
 
 // Where row m's operands start in ua and ub, in floats. Plain rows (w = 0): m ld_in in both. Rows of
 // the pair basis (w node pairs, nq basis rows per leaf, n leaves; see leaf_pair_level_kernel):
@@ -57,88 +56,137 @@ struct MergeRows {
   }
 };
 
-__global__ void __launch_bounds__(256, 2)
+// A workgroup owns one group i, all 32 outputs j and 128 rows, 32 a wave. 160 registers leave three
+// workgroups on a CU (two blocks of rows a wave share the T_i operands but need every register and
+// spill: 375 against 246 us at 16384 rows, G = 48).
+__global__ void __launch_bounds__(256, 3)
 quadrilinear_merge_kernel(const float* __restrict__ T, const float* __restrict__ ua, const float* __restrict__ ub,
                           float* __restrict__ out, int64_t M, int G, MergeRows rows) {
-  __shared__ float Ts[kQKL * kQHalf];  // Ts[kl][jj] = T[i][16 jh + jj][k][l], kl = 32 k + l
+  // [buffer][k][part][l half-block s][64 chunks of 8 l]: chunk (j, h) of block (k, s) at
+  // 2 j + (h ^ (j / 4 mod 2)) + (2 k + s), mod 64, which spreads both the eight blocks a row's
+  // stores go to and any 8 consecutive lanes of a read over the banks
+  __shared__ v4u Ts[2][kQK][3][2][64];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 4, c = lane & 15;
+  const int hh = lane >> 5, c = lane & 31;
   const int i = blockIdx.y;
-  const int jh = blockIdx.z;
-  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kQRows + wave * 64;
+  const int64_t m0 = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * 32;
   const int64_t ld = static_cast<int64_t>(G) * kQR;  // floats per row of out
 
-  // stage T_i's half: thread t takes output jj = t mod 16 and 4 consecutive kl per pass
-  const float* Ti = T + (static_cast<int64_t>(i) * kQR + kQHalf * jh) * kQKL;
-  for (int base = 0; base < kQKL * kQHalf / 4; base += 256) {
-    const int it = base + tid;
-    const int jj = it & 15, kl4 = it >> 4;
-    const float4 v = *reinterpret_cast<const float4*>(Ti + static_cast<int64_t>(jj) * kQKL + 4 * kl4);
-    Ts[(4 * kl4 + 0) * kQHalf + jj] = v.x;
-    Ts[(4 * kl4 + 1) * kQHalf + jj] = v.y;
-    Ts[(4 * kl4 + 2) * kQHalf + jj] = v.z;
-    Ts[(4 * kl4 + 3) * kQHalf + jj] = v.w;
-  }
-
-  // this lane's rows (one per 16-row tile): all 32 values of a, and b at l = 4 m + g
-  float a[4][kQR], b[4][8];
+  // staging: thread t takes 16 consecutive l of (j = t / 8, k = t / 2 mod 4)
+  const int sj = tid >> 3, sk = (tid >> 1) & 3, ss = tid & 1;
+  const float* Tp = T + ((static_cast<int64_t>(i) * kQR + sj) * kQR + sk) * kQR + 16 * ss;
+  float4 rt[4];
+  auto tload = [&](int k0) {
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt) {
-    const int64_t row = row0 + 16 * rt + c;
-    const bool ok = row < M;
-    int64_t ao, bo;
-    rows.at(ok ? row : 0, ao, bo);
-    const float* ar = ua + ao + i * kQR;
-    const float* br = ub + bo + i * kQR;
+    for (int u = 0; u < 4; ++u) rt[u] = *reinterpret_cast<const float4*>(Tp + k0 * kQR + 4 * u);
+  };
+  auto tstore = [&](int buf) {
 #pragma unroll
-    for (int q = 0; q < kQR / 4; ++q) {
-      const float4 v = ok ? *reinterpret_cast<const float4*>(ar + 4 * q) : make_float4(0.f, 0.f, 0.f, 0.f);
-      a[rt][4 * q] = v.x;
-      a[rt][4 * q + 1] = v.y;
-      a[rt][4 * q + 2] = v.z;
-      a[rt][4 * q + 3] = v.w;
+    for (int h = 0; h < 2; ++h) {
+      const float x[8] = {rt[2 * h].x,     rt[2 * h].y,     rt[2 * h].z,     rt[2 * h].w,
+                          rt[2 * h + 1].x, rt[2 * h + 1].y, rt[2 * h + 1].z, rt[2 * h + 1].w};
+      const Split8 sp = split8(x);
+      const int slot = (2 * sj + (h ^ ((sj >> 2) & 1)) + 2 * sk + ss) & 63;
+      Ts[buf][sk][0][ss][slot] = sp.h;
+      Ts[buf][sk][1][ss][slot] = sp.m;
+      Ts[buf][sk][2][ss][slot] = sp.l;
     }
+  };
+
+  // this lane's row (past M the last): b split once, four values of a a chunk
+  const int64_t row = m0 + c;
+  int64_t ao, bo;
+  rows.at(row < M ? row : M - 1, ao, bo);
+  const float* const ar = ua + ao + i * kQR;
+  const float* const br = ub + bo + i * kQR;
+  bf16x8 bs[2][3];
+  tload(0);
 #pragma unroll
-    for (int m = 0; m < 8; ++m) b[rt][m] = ok ? br[4 * m + g] : 0.f;
+  for (int s = 0; s < 2; ++s) {
+    const float4 v0 = *reinterpret_cast<const float4*>(br + 16 * s + 8 * hh);
+    const float4 v1 = *reinterpret_cast<const float4*>(br + 16 * s + 8 * hh + 4);
+    const float x[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+    const Split8 sp = split8(x);
+    bs[s][0] = as_bf16x8(sp.h);
+    bs[s][1] = as_bf16x8(sp.m);
+    bs[s][2] = as_bf16x8(sp.l);
   }
+  v4f av = *reinterpret_cast<const v4f*>(ar);
+  tstore(0);
   __syncthreads();
 
-  // step t contracts kl = 4 t + g, i.e. k = t / 8, l = 4 (t mod 8) + g
-  v4f acc[4];
-#pragma unroll
-  for (int rt = 0; rt < 4; ++rt) acc[rt] = zero4();
-#pragma unroll
-  for (int k = 0; k < kQR; ++k) {
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-      const float tb = Ts[(32 * k + 4 * m + g) * kQHalf + c];
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) acc[rt] = mfma16x4(a[rt][k] * b[rt][m], tb, acc[rt]);
+  v16f acc = v16f{};
+  const int slot0 = 2 * c + (hh ^ ((c >> 2) & 1));
+#pragma unroll 1
+  for (int ch = 0; ch < kQR / kQK; ++ch) {
+    const int buf = ch & 1;
+    const bool more = ch + 1 < kQR / kQK;
+    v4f an = av;
+    if (more) {
+      tload((ch + 1) * kQK);
+      an = *reinterpret_cast<const v4f*>(ar + (ch + 1) * kQK);
     }
+#pragma unroll
+    for (int k = 0; k < kQK; ++k) {
+      v16f w = v16f{};
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int slot = (slot0 + 2 * k + s) & 63;
+        bf16x8 t[3];
+#pragma unroll
+        for (int part = 0; part < 3; ++part) t[part] = as_bf16x8(Ts[buf][k][part][s][slot]);
+#pragma unroll
+        for (int e = 0; e < kSplitTerms; ++e) w = mfma32_bf16(t[kSplitA[e]], bs[s][kSplitB[e]], w);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[e] = fmaf(w[e], av[k], acc[e]);
+    }
+    if (more) tstore(buf ^ 1);
+    av = an;
+    __syncthreads();
   }
 
-  // lane (g, c) holds out[row0 + 16 rt + 4 g + r][i R + 16 jh + c]
+  // element e: output j = 8 (e / 4) + 4 hh + e % 4 of row m0 + c
+  bool bad = false;
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
+  for (int e = 0; e < 16; ++e) bad |= !finite_f32(acc[e]);
+  if (__any(bad)) {  // formed again in float32 (through LDS: an index known at run time)
+    float* const mine = reinterpret_cast<float*>(&Ts[0][0][0][0][0]) + wave * 1024 + lane;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t row = row0 + 16 * rt + 4 * g + r;
-      if (row < M) out[row * ld + i * kQR + kQHalf * jh + c] = acc[rt][r];
+    for (int e = 0; e < 16; ++e) mine[64 * e] = acc[e];
+#pragma unroll 1
+    for (int e = 0; e < 16; ++e) {
+      if (finite_f32(mine[64 * e]) || row >= M) continue;
+      const float* tj = T + (static_cast<int64_t>(i) * kQR + 8 * (e >> 2) + 4 * hh + (e & 3)) * kQR * kQR;
+      float v = 0.f;
+#pragma unroll 1
+      for (int kl = 0; kl < kQR * kQR; ++kl) v = fmaf(ar[kl >> 5] * br[kl & 31], tj[kl], v);
+      mine[64 * e] = v;
     }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = mine[64 * e];
+  }
+  if (row < M) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<v4f*>(out + row * ld + i * kQR + 8 * q + 4 * hh) =
+          v4f{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+  }
 }
 
 // --------------------------------------------------------------------------------------
 // Tiled GEMM with epilogues
 // --------------------------------------------------------------------------------------
 constexpr int kBM = 128, kBN = 128, kBK = 16;
-// Row lengths of As[k][row] and Bs[k][col] (floats): 16 more than a tile, so the four k rows
-// of one operand read (lanes 16 g + c read row g, column c) fall on distinct banks. A's
-// transposed stores put column r of k rows 4q .. 4q + 3 at r ^ 16 q, so the four lanes that
-// share r (q = 0..3, rows 4 x 144 floats apart, one bank) write four banks; a read's four
+// Row lengths of gemm_rows_f32_kernel's As[k][row] and Bs[k][col] (floats): 16 more than a tile,
+// so the four k rows of one operand read (lanes 16 g + c read row g, column c) fall on distinct
+// banks. A's transposed stores put column r of k rows 4q .. 4q + 3 at r ^ 16 q, so the four lanes
+// that share r (q = 0..3, rows 4 x 144 floats apart, one bank) write four banks; a read's four
 // rows share q, so it still covers one aligned 16-column block per row.
-constexpr int kAPad = kBM + 16;
 constexpr int kBPad = kBN + 16;
+
+constexpr int kAhead = 2;  // K slices in flight in registers (even)
 
 enum GemmEpi { kEpiPlain = 0, kEpiCond = 1, kEpiResidual = 2, kEpiRowMask = 3 };
 
@@ -147,12 +195,21 @@ enum GemmEpi { kEpiPlain = 0, kEpiCond = 1, kEpiResidual = 2, kEpiRowMask = 3 };
 // row range, nonzero when the rows are processed in chunks); kEpiResidual adds res[m, n];
 // kEpiRowMask multiplies row m by (mask[m] != 0), aux then being a uint8 mask.
 // C may be the residual itself (each output entry reads its residual entry, then overwrites
-// it, in one thread), so neither carries __restrict__. VEC: K and N are multiples of 4
-// (16-byte staging loads); otherwise the staging loads are per element.
+// it, in one thread), so neither carries __restrict__. VEC: K is a multiple of 4 (16-byte loads
+// of A); otherwise those loads are per element.
 // Split K (gridDim.z > 1): workgroup z contracts k in [z K, min(z K + K, Ktot)) of A (row
 // stride lda) and B and writes its partial product (EPI plain) at C + z cz.
+//
+// float32 products as six bfloat16 products (split_f32.h), K slices of 16 (one matrix step). A
+// workgroup owns 128 rows x 128 columns, a wave 32 rows and every column: its rows of A go from
+// memory to the wave's registers (8 consecutive k per lane, split there, so no two waves split
+// the same row), the slice's columns of B through LDS, double-buffered, as their three bfloat16
+// parts: a column is 2 chunks of 8 k (16 bytes, one operand read), chunk h of column n at
+// h ^ ((n / 4) mod 2), which spreads any 8 consecutive lanes of a read or a store over all banks.
+// A thread stages 8 k of one column. Loads run kAhead slices ahead of their products (1024 rows,
+// one workgroup to a CU: 202 us with one slice, 166 with two, 167 with four).
 template <int EPI, bool VEC>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, 3)
 gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ Bm, float* C, const float* aux, int64_t M, int N,
                 int K, int h_rows, int64_t row0, int lda, int Ktot, int64_t cz) {
   {
@@ -162,111 +219,143 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ Bm, float
     C += static_cast<int64_t>(blockIdx.z) * cz;
     K = Ktot - kbeg < K ? Ktot - kbeg : K;
   }
-  __shared__ float As[2][kBK][kAPad];
-  __shared__ float Bs[2][kBK][kBPad];
+  constexpr int kPart = 2 * kBN;  // 16-byte chunks of one part of B's slice
+  __shared__ v4u smem[2][3 * kPart];
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 4, c = lane & 15;
-  const int64_t m0 = static_cast<int64_t>(blockIdx.y) * kBM;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hh = lane >> 5, c = lane & 31;
+  const int64_t m0 = static_cast<int64_t>(blockIdx.y) * kBM + wave * 32;
   const int n0 = blockIdx.x * kBN;
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;  // this wave's 64 x 64 sub-tile
 
-  // global -> register staging: A tile 128 x 16 as 512 float4 (row = it / 4, k4 = it % 4),
-  // B tile 16 x 128 as 512 float4 (k = it / 32, n4 = it % 32); two of each per thread
-  float4 ra[2], rb[2];
-  auto gload = [&](int k0) {
+  // Rows and columns past the matrix repeat its last (their sums are not stored).
+  const float* const Ap = A + (m0 + c < M ? m0 + c : M - 1) * lda + 8 * hh;
+  const int bc = tid & 127, bh = wave >> 1;  // this thread's column and k half of B's slice
+  const int bn = n0 + bc < N ? n0 + bc : N - 1;
+  const int bslot = 2 * bc + (bh ^ ((bc >> 2) & 1));
+  float ra[kAhead][8], rb[kAhead][8];
+  // a whole slice: no bounds, so nothing waits for these loads before they are staged
+  auto gload = [&](int k0, float (&ra)[8], float (&rb)[8]) {
+    if constexpr (VEC) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int it = tid + 256 * u;
-      const int64_t row = m0 + (it >> 2);
-      const int kk = k0 + 4 * (it & 3);
-      if constexpr (VEC) {
-        ra[u] = (row < M && kk < K) ? *reinterpret_cast<const float4*>(A + row * lda + kk)
-                                    : make_float4(0.f, 0.f, 0.f, 0.f);
-      } else {
-        const float* ar = A + (row < M ? row : 0) * lda;
-        ra[u].x = (row < M && kk < K) ? ar[kk] : 0.f;
-        ra[u].y = (row < M && kk + 1 < K) ? ar[kk + 1] : 0.f;
-        ra[u].z = (row < M && kk + 2 < K) ? ar[kk + 2] : 0.f;
-        ra[u].w = (row < M && kk + 3 < K) ? ar[kk + 3] : 0.f;
+      for (int u = 0; u < 2; ++u) {
+        const v4f v = *reinterpret_cast<const v4f*>(Ap + k0 + 4 * u);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ra[4 * u + i] = v[i];
       }
-      const int kb = k0 + (it >> 5);
-      const int nn = n0 + 4 * (it & 31);
-      if constexpr (VEC) {
-        rb[u] = (kb < K && nn < N) ? *reinterpret_cast<const float4*>(Bm + static_cast<int64_t>(kb) * N + nn)
-                                   : make_float4(0.f, 0.f, 0.f, 0.f);
-      } else {
-        const float* br = Bm + static_cast<int64_t>(kb < K ? kb : 0) * N;
-        rb[u].x = (kb < K && nn < N) ? br[nn] : 0.f;
-        rb[u].y = (kb < K && nn + 1 < N) ? br[nn + 1] : 0.f;
-        rb[u].z = (kb < K && nn + 2 < N) ? br[nn + 2] : 0.f;
-        rb[u].w = (kb < K && nn + 3 < N) ? br[nn + 3] : 0.f;
-      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) ra[u] = Ap[k0 + u];
+    }
+    const float* const bk = Bm + static_cast<int64_t>(k0 + 8 * bh) * N;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) rb[u] = (bk + static_cast<int64_t>(u) * N)[bn];
+  };
+  // the last slice where K is not a multiple of 16, zeros past K
+  auto gload_tail = [&](int k0, float (&ra)[8], float (&rb)[8]) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int ka = k0 + 8 * hh + u, kb = k0 + 8 * bh + u;
+      ra[u] = ka < K ? Ap[k0 + u] : 0.f;
+      rb[u] = kb < K ? Bm[static_cast<int64_t>(kb) * N + bn] : 0.f;
     }
   };
-  auto sstore = [&](int buf) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int it = tid + 256 * u;
-      const int r = it >> 2, k4 = 4 * (it & 3);
-      // column r of rows k4 .. k4 + 3 at r ^ 16 ((k4 / 4) mod 4): the four lanes sharing r
-      // (k4 = 0, 4, 8, 12) land in four banks instead of one
-      const int rs = r ^ (16 * ((k4 >> 2) & 3));
-      As[buf][k4 + 0][rs] = ra[u].x;
-      As[buf][k4 + 1][rs] = ra[u].y;
-      As[buf][k4 + 2][rs] = ra[u].z;
-      As[buf][k4 + 3][rs] = ra[u].w;
-      *reinterpret_cast<float4*>(&Bs[buf][it >> 5][4 * (it & 31)]) = rb[u];
-    }
+  bf16x8 af[3];
+  auto stage = [&](int buf, const float (&ra)[8], const float (&rb)[8]) {
+    const Split8 sa = split8(ra), sb = split8(rb);
+    af[0] = as_bf16x8(sa.h);
+    af[1] = as_bf16x8(sa.m);
+    af[2] = as_bf16x8(sa.l);
+    smem[buf][bslot] = sb.h;
+    smem[buf][kPart + bslot] = sb.m;
+    smem[buf][2 * kPart + bslot] = sb.l;
   };
 
-  v4f acc[4][4];
+  constexpr int NT = kBN / 32;
+  v16f acc[NT];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = zero4();
+  for (int nt = 0; nt < NT; ++nt) acc[nt] = v16f{};
 
-  const int nk = (K + kBK - 1) / kBK;
-  gload(0);
-  sstore(0);
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < nk) gload((kt + 1) * kBK);
+  const int rd = 2 * c + (hh ^ ((c >> 2) & 1));  // this lane's chunk of column c of a block
+  auto products = [&](int buf) {
 #pragma unroll
-    for (int ks = 0; ks < kBK; ks += 4) {
-      float af[4], bf[4];
+    for (int nt = 0; nt < NT; ++nt) {
+      bf16x8 bf[3];
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt) af[mt] = As[buf][ks + g][(wm + 16 * mt + c) ^ (16 * ((ks >> 2) & 3))];
+      for (int part = 0; part < 3; ++part) bf[part] = as_bf16x8(smem[buf][part * kPart + 64 * nt + rd]);
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) bf[nt] = Bs[buf][ks + g][wn + 16 * nt + c];
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = mfma16x4(af[mt], bf[nt], acc[mt][nt]);
+      for (int s = 0; s < kSplitTerms; ++s) acc[nt] = mfma32_bf16(af[kSplitA[s]], bf[kSplitB[s]], acc[nt]);
     }
-    if (kt + 1 < nk) sstore(buf ^ 1);
+  };
+  // Slice kt in LDS buffer kt mod 2 and, on its way there, register set kt mod kAhead; loads past
+  // the last whole slice repeat it.
+  const int nf = K / kBK;
+  if (nf > 0) {
+    auto at = [&](int kt) { return (kt < nf ? kt : nf - 1) * kBK; };
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) gload(at(j), ra[j], rb[j]);
+    stage(0, ra[0], rb[0]);
     __syncthreads();
-  }
-
-  // lane (g, c) holds C[wm + 16 mt + 4 g + r][wn + 16 nt + c]
+    for (int kt = 0; kt < nf; kt += kAhead) {
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t row = m0 + wm + 16 * mt + 4 * g + r;
-      if (row >= M) continue;
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        const int col = n0 + wn + 16 * nt + c;
-        if (col >= N) continue;
-        float v = acc[mt][nt][r];
-        if constexpr (EPI == kEpiCond) v *= aux[((row0 + row) % h_rows) * N + col];
-        if constexpr (EPI == kEpiResidual) v += aux[row * N + col];
-        if constexpr (EPI == kEpiRowMask) v *= reinterpret_cast<const uint8_t*>(aux)[row] != 0 ? 1.f : 0.f;
-        C[row * N + col] = v;
+      for (int j = 0; j < kAhead; ++j) {
+        if (kt + j == nf) break;
+        gload(at(kt + j + kAhead), ra[j], rb[j]);
+        products(j & 1);
+        stage((j + 1) & 1, ra[(j + 1) % kAhead], rb[(j + 1) % kAhead]);
+        __syncthreads();
       }
     }
+  }
+  if (nf * kBK < K) {
+    gload_tail(nf * kBK, ra[0], rb[0]);
+    stage(0, ra[0], rb[0]);
+    __syncthreads();
+    products(0);
+  }
+  __syncthreads();  // smem is free for the epilogue
+
+  // element i of block nt: row m0 + 8 (i / 4) + 4 hh + i % 4, column n0 + 32 nt + c
+  auto row_of = [&](int i) { return m0 + 8 * (i >> 2) + 4 * hh + (i & 3); };
+  float* const mine = reinterpret_cast<float*>(&smem[0][0]) + wave * 1024 + lane;
+  unsigned hrow[16];
+  if constexpr (EPI == kEpiCond) {
+    const unsigned hbase = static_cast<unsigned>((row0 + m0) % h_rows);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) hrow[i] = (hbase + static_cast<unsigned>(row_of(i) - m0)) % static_cast<unsigned>(h_rows);
+  }
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int col = n0 + 32 * nt + c;
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) bad |= !finite_f32(acc[nt][i]);
+    if (__any(bad)) {  // formed again in float32 (through LDS: an index known at run time)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mine[64 * i] = acc[nt][i];
+#pragma unroll 1
+      for (int i = 0; i < 16; ++i) {
+        const int64_t row = row_of(i);
+        if (finite_f32(mine[64 * i]) || row >= M || col >= N) continue;
+        float v = 0.f;
+#pragma unroll 1
+        for (int k = 0; k < K; ++k) v = fmaf(A[row * lda + k], Bm[static_cast<int64_t>(k) * N + col], v);
+        mine[64 * i] = v;
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[nt][i] = mine[64 * i];
+    }
+    if (col >= N) continue;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int64_t row = row_of(i);
+      if (row >= M) continue;
+      float v = acc[nt][i];
+      if constexpr (EPI == kEpiCond) v *= aux[static_cast<int64_t>(hrow[i]) * N + col];
+      if constexpr (EPI == kEpiResidual) v += aux[row * N + col];
+      if constexpr (EPI == kEpiRowMask) v *= reinterpret_cast<const uint8_t*>(aux)[row] != 0 ? 1.f : 0.f;
+      C[row * N + col] = v;
+    }
+  }
 }
 
 // Site-masked product C[m, :] = mask[m] != 0 ? A[m, :] B : 0 with the masked rows skipped.
@@ -477,18 +566,28 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* __restr
   *reinterpret_cast<float4*>(C + 4 * i4) = v;
 }
 
+// One launch; parts > 1: split K.
+template <int EPI>
+hipError_t launch_tiles(const float* A, const float* B, float* C, const float* aux, int64_t M, int N, int kp, int parts,
+                        int h_rows, int64_t row0, int K, int64_t cz, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>((N + kBN - 1) / kBN), static_cast<unsigned>((M + kBM - 1) / kBM),
+                  static_cast<unsigned>(parts));
+  auto kern = K % 4 == 0 ? gemm_f32_kernel<EPI, true> : gemm_f32_kernel<EPI, false>;
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, A, B, C, aux, M, N, kp, h_rows, row0, K, K, cz);
+  return hipGetLastError();
+}
+
 template <int EPI>
 hipError_t launch_gemm(const float* A, const float* B, float* C, const float* aux, int64_t M, int N, int K,
                        int h_rows, int64_t row0, hipStream_t stream, float* split_ws = nullptr,
                        int64_t split_cap = 0) {
-  const dim3 grid(static_cast<unsigned>((N + kBN - 1) / kBN), static_cast<unsigned>((M + kBM - 1) / kBM));
   // Split K where the tiles leave most CUs idle (the tree's deep levels: 1024-4096 rows,
   // 64-512 tiles of 96-step K chains): S parts of K into split_ws [S, M, N], then one pass
   // that sums the parts in order and applies the epilogue (deterministic).
   if (split_ws != nullptr && N % 4 == 0 && K % 4 == 0 && K >= 256) {
     int cus = 0;
     if (hipError_t err = device_cu_count(&cus); err != hipSuccess) return err;
-    const int64_t tiles = static_cast<int64_t>(grid.x) * grid.y;
+    const int64_t tiles = static_cast<int64_t>((N + kBN - 1) / kBN) * ((M + kBM - 1) / kBM);
     const int64_t mn = M * N;
     int64_t S = tiles < cus ? (2 * cus + tiles - 1) / tiles : 1;
     S = S > 8 ? 8 : S;
@@ -497,23 +596,16 @@ hipError_t launch_gemm(const float* A, const float* B, float* C, const float* au
     if (S >= 2) {
       const int kp = static_cast<int>(((K + S - 1) / S + kBK - 1) / kBK * kBK);
       const int parts = (K + kp - 1) / kp;
-      const dim3 gs(grid.x, grid.y, static_cast<unsigned>(parts));
-      hipLaunchKernelGGL((gemm_f32_kernel<kEpiPlain, true>), gs, dim3(256), 0, stream, A, B, split_ws, nullptr, M, N,
-                         kp, 1, int64_t(0), K, K, mn);
-      if (hipError_t err = hipGetLastError(); err != hipSuccess) return err;
+      if (hipError_t err = launch_tiles<kEpiPlain>(A, B, split_ws, nullptr, M, N, kp, parts, 1, 0, K, mn, stream);
+          err != hipSuccess)
+        return err;
       const int64_t n4 = mn / 4;
       hipLaunchKernelGGL((splitk_reduce_kernel<EPI>), dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0,
                          stream, split_ws, C, aux, M, N, parts, mn, h_rows, row0);
       return hipGetLastError();
     }
   }
-  if (N % 4 == 0 && K % 4 == 0)
-    hipLaunchKernelGGL((gemm_f32_kernel<EPI, true>), grid, dim3(256), 0, stream, A, B, C, aux, M, N, K, h_rows, row0,
-                       K, K, int64_t(0));
-  else
-    hipLaunchKernelGGL((gemm_f32_kernel<EPI, false>), grid, dim3(256), 0, stream, A, B, C, aux, M, N, K, h_rows,
-                       row0, K, K, int64_t(0));
-  return hipGetLastError();
+  return launch_tiles<EPI>(A, B, C, aux, M, N, K, 1, h_rows, row0, K, 0, stream);
 }
 
 // One factorized apply over rows [row0, row0 + M) of the caller's range: x, residual and y
@@ -795,7 +887,7 @@ bool basis_serves(int64_t B, int n, int nq) {
 
 hipError_t launch_merge(const float* T, const float* ua, const float* ub, float* out, int64_t M, int G,
                         const MergeRows& rows, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>((M + kQRows - 1) / kQRows), static_cast<unsigned>(G), 2);
+  const dim3 grid(static_cast<unsigned>((M + 127) / 128), static_cast<unsigned>(G));
   hipLaunchKernelGGL(quadrilinear_merge_kernel, grid, dim3(256), 0, stream, T, ua, ub, out, M, G, rows);
   return hipGetLastError();
 }

@@ -91,6 +91,57 @@ def test_factorized_apply(walkers, nodes, d_in, R, d_out, residual):
     assert rel(got.cpu().numpy(), want) <= TOL
 
 
+@pytest.mark.parametrize("M,d_in,R,d_out", [(1, 1, 1, 1), (127, 15, 16, 129), (129, 17, 33, 2), (128, 16, 32, 128), (5, 4, 260, 131)])
+def test_factorized_apply_tile_edges(M, d_in, R, d_out):
+    """One row, column or k either side of the 128 x 128 tiles and 16-deep slices; large and tiny
+    magnitudes beside each other (each factor's terms keep their float32 bits: same bound)."""
+    from hamiltonzero_amd import executor
+
+    _say(f"apply edges M={M} d_in={d_in} R={R} d_out={d_out}")
+    rng = np.random.default_rng(M + 3 * d_in + R)
+    x = (rng.standard_normal((M, d_in)) * 10.0 ** rng.integers(-6, 7, size=(M, 1))).astype(np.float32)
+    V, U = rng.standard_normal((d_in, R)).astype(np.float32), rng.standard_normal((R, d_out)).astype(np.float32)
+    h = rng.standard_normal((1, R)).astype(np.float32)
+    got = executor._factorized_apply(types.SimpleNamespace(V=dev(V), U=dev(U)), dev(h), dev(x)).cpu().numpy()
+    want = X.factorized_apply(V, U, h, x)
+    # per row: a float32 sum's bound scales with the sum of its terms' magnitudes
+    terms = ((np.abs(x.astype(np.float64)) @ np.abs(V)) * np.abs(h)) @ np.abs(U)
+    assert np.all(np.abs(got - want) <= 2.0**-24 * (d_in + R + 4) ** 0.5 * 4 * terms)
+
+
+def test_products_of_values_the_split_does_not_hold():
+    """Infinities, NaN and finite values above the largest bfloat16 (3.39e38): the sums are what
+    float32 arithmetic gives, and only in the rows (and groups) that hold such a value."""
+    from hamiltonzero_amd import executor
+
+    _say("apply and merge, non-finite and largest values")
+    rng = np.random.default_rng(3)
+    M, d = 40, 48
+    x = rng.random((M, d)).astype(np.float32) + 0.5
+    V, U = (rng.random((d, d)).astype(np.float32) * 1e-3 + 1e-3 for _ in range(2))
+    h = np.ones((1, d), np.float32)
+    x[3, 7], x[9, 0], x[20, 40], x[33, 5] = np.inf, np.nan, 3.4e38, -np.inf
+    fac = types.SimpleNamespace(V=dev(V), U=dev(U))
+    got = executor._factorized_apply(fac, dev(h), dev(x)).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        want = X.factorized_apply(V, U, h, x)
+    assert np.all(np.isposinf(got[3])) and np.all(np.isneginf(got[33])) and np.all(np.isnan(got[9]))
+    ok = [m for m in range(M) if m not in (3, 9, 33)]
+    assert np.all(np.abs(got[ok] - want[ok]) <= TOL * np.abs(want[ok]))  # every term is positive
+
+    G, R = 2, 32
+    T = rng.random((G, R, R, R)).astype(np.float32)
+    a, b = (rng.random((M, G * R)).astype(np.float32) + 0.5 for _ in range(2))
+    a[3, 5], b[9, 40], a[20, 33], b[33, 1] = np.inf, np.nan, 3.4e38, -np.inf
+    b[20] *= 1e-6
+    got = executor.quadrilinear_merge(dev(T), dev(a), dev(b)).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        want = X.quadrilinear_merge(T, a, b)
+    assert np.all(np.isposinf(got[3, :R])) and np.all(np.isnan(got[9, R:])) and np.all(np.isneginf(got[33, :R]))
+    mask = np.isfinite(want)
+    assert np.all(np.isfinite(got) == mask) and np.all(np.abs(got[mask] - want[mask]) <= TOL * np.abs(want[mask]))
+
+
 def test_merge_level_products_compose():
     """One tree level's products as the executor chains them: merge, then the residual apply
     (execute.py:103-104), checked against the oracle's level up to the RMS rescale."""
