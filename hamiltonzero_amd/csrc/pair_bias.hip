@@ -1,5 +1,5 @@
-// The trunk attention's coupling-bias producer on the float32 matrix cores
-// (v_mfma_f32_16x16x4_f32): per site pair (i, j) of a walker,
+// The trunk attention's coupling-bias producer, float32 products as six bfloat16 ones
+// (split_f32.h, v_mfma_f32_16x16x32_bf16): per site pair (i, j) of a walker,
 //     y   = x * (w * rsqrt(mean(x^2) + eps))           x = edge[b, i, j, :] (C channels)
 //     h0  = y W_in + b_in                               (64 hidden)
 //     h1  = h0 + gain * (silu(h0 W_1 + b_1) W_2 + b_2)
@@ -12,48 +12,61 @@
 //
 // Orientation: every layer is computed transposed, features x pairs (features = the 16-row
 // M blocks, 16 pairs = one N block), so the pairs are the columns of the B operand and the
-// weights (staged once per workgroup in LDS, as ready-made A fragments) the A operand. A
-// layer's result C[feature 4g + r][pair c] sits in lane (g, c) register r, which is exactly
-// the B operand the next layer needs if that layer's K order is permuted: K step (kb, r) of
-// lane group g multiplies feature 16 kb + 4 g + r. The weight fragments are stored in that
-// order, so the four layers chain in registers with no LDS round trip.
+// weights (split once per workgroup into LDS, as ready-made A fragments) the A operand. A
+// layer's result C[feature 4g + r][pair c] of block m sits in lane (g, c) register r, and the two
+// blocks 2s, 2s + 1 are exactly the eight values of the next layer's B operand in K step s if that
+// layer's K order is permuted: slot j of lane group g multiplies feature 32 s + 16 (j / 4) + 4 g +
+// j mod 4. The weight fragments are stored in that order, so the four layers chain in registers,
+// split between layers, with no LDS round trip.
 //
-// The RMS scale r is a per-pair (column) scale: layer 1 runs on x * w and scales columns by r
-// afterwards, so x streams straight from memory into the products while mean(x^2) (and,
-// with a tangent, mean(x xdot)) accumulate alongside; the tangent of layer 1 is
-// r (xdot * w) W_in + rdot (x * w) W_in with rdot = -0.5 r / v * 2 mean(x xdot).
+// The RMS scale r is a per-pair (column) scale and the norm weight w is folded into W_in's
+// fragments: layer 1 runs on x and scales columns by r afterwards, so x streams straight from
+// memory into the products while mean(x^2) (and, with a tangent, mean(x xdot)) accumulate
+// alongside; the tangent of layer 1 is r xdot (w W_in) + rdot x (w W_in) with rdot = -0.5 r / v *
+// 2 mean(x xdot).
+//
+// The weights' three parts (98 KB at C = 96, 32 heads) leave one workgroup per CU, of eight
+// waves: two a SIMD, so one wave's splits and activations run under the other's products. A tile's
+// 384 matrix instructions take 6144 cycles beside about 1400 vector instructions (5600 cycles);
+// with two waves a SIMD they overlap by a third. 1024 walkers of 36 sites, C = 96, 32 heads, with
+// tangent: 495 us (760 on the float32 matrix instruction); 250 us of that with neither the products
+// nor memory, 90 us for the products beyond it, 95 us for the loads and stores. Twelve waves spill
+// and take 545 us.
 //
 // A tile is 16 pairs with their tangent (T = 1: N block 0 primal, N block 1 tangent) or 32
 // pairs (T = 0). With a mask, only pairs whose key site is physical are computed (and, in
 // the square-mask semantics, whose query site is physical too): a wave builds the walker's
 // list of physical sites with a ballot, then walks the flattened (query, key) pair list.
-// Each wave is persistent over (walker, part) items; a workgroup's four waves share the
-// staged weights.
+// Each wave is persistent over (walker, part) items; a workgroup's waves share the staged weights.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "mhsea_device.h"
 #include "mhsea_launch.h"
+#include "split_f32.h"
 
 namespace hz {
 namespace {
 
 constexpr int kHid = 64;          // bias_mlp hidden width (trunk_attention_bias_hidden_dim)
-constexpr int kPBWaves = 4;       // waves per workgroup
+constexpr int kPBWaves = 8;       // waves per workgroup
 constexpr int kPBListN = 256;     // sites per walker the pair compaction handles
 
 template <int C, int HB>
 struct PBLds {
-  static constexpr int kF1 = 0;                  // W_in fragments: 4 M blocks x C/4 K steps x 64 lanes
-  static constexpr int kF2 = kF1 + 64 * C;       // W_1 fragments: 4 x 16 x 64
-  static constexpr int kF3 = kF2 + 4096;         // W_2 fragments
-  static constexpr int kF4 = kF3 + 4096;         // W_out fragments: HB x 16 x 64
-  static constexpr int kBin = kF4 + 1024 * HB;
+  // fragments, 16-byte units: [K step][M block][part][64 lanes]
+  static constexpr int kBlock = 3 * 64;
+  static constexpr int kF1 = 0;                            // W_in: C / 32 steps x 4 blocks
+  static constexpr int kF2 = kF1 + C / 32 * 4 * kBlock;    // W_1: 2 x 4
+  static constexpr int kF3 = kF2 + 8 * kBlock;             // W_2
+  static constexpr int kF4 = kF3 + 8 * kBlock;             // W_out: 2 x HB
+  static constexpr int kUnits = kF4 + 2 * HB * kBlock;
+  // vectors, floats
+  static constexpr int kBin = 0;
   static constexpr int kB1 = kBin + kHid;
   static constexpr int kB2 = kB1 + kHid;
   static constexpr int kBout = kB2 + kHid;
-  static constexpr int kLnw = kBout + 16 * HB;
-  static constexpr int kFloats = kLnw + C;
+  static constexpr int kFloats = kBout + 16 * HB;
 };
 
 __device__ __forceinline__ float4 lds4(const float* base, int off) {
@@ -106,48 +119,61 @@ __device__ __forceinline__ void load_rows(const float* edge_b, const float* edge
   }
 }
 
-// Workgroups per CU: two while the staged weights and the wave lists fit half of the LDS
-// (every instantiation but C = 128 with 64 heads, whose weights take 83.5 KB), else one.
-template <int C, int HB>
-constexpr int pb_occupancy() {
-  return (PBLds<C, HB>::kFloats * 4 + kPBWaves * kPBListN * 2) <= 80 * 1024 ? 2 : 1;
+// Splits one layer's weights into its fragments: w(k, o) the weight, k_of(step, g, j) the K order.
+template <int KS, int MB, class W, class K>
+__device__ __forceinline__ void stage_frags(v4u* dst, W w, K k_of) {
+  for (int f = threadIdx.x; f < KS * MB * 64; f += blockDim.x) {
+    const int lane = f & 63, m = (f >> 6) % MB, step = (f >> 6) / MB;
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = w(k_of(step, lane >> 4, j), 16 * m + (lane & 15));
+    const Split8 sp = split8(x);
+    v4u* const d = dst + (step * MB + m) * (3 * 64) + lane;
+    d[0] = sp.h;
+    d[64] = sp.m;
+    d[128] = sp.l;
+  }
+}
+
+// out[m][cb] += W x[.][cb] over 64 features, the layers' registers as they stand.
+template <int MB>
+__device__ __forceinline__ void hidden_layer(const v4u* F, const v4f (&x)[4][2], v4f (&out)[MB][2]) {
+#pragma unroll
+  for (int step = 0; step < 2; ++step) {
+    float x0[8], x1[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      x0[j] = x[2 * step + (j >> 2)][0][j & 3];
+      x1[j] = x[2 * step + (j >> 2)][1][j & 3];
+    }
+    mm_step<MB>(F + step * MB * (3 * 64), split8(x0), split8(x1), out);
+  }
 }
 
 template <int C, int HB, bool TAN>
-__global__ void __launch_bounds__(256, (pb_occupancy<C, HB>())) pair_bias_kernel(PairBiasParams p) {
+__global__ void __launch_bounds__(64 * kPBWaves, 2) pair_bias_kernel(PairBiasParams p) {
   using L = PBLds<C, HB>;
-  constexpr int C4 = C / 4;    // channels per lane group = layer-1 K steps
+  constexpr int C4 = C / 4;    // channels per lane group
   constexpr int CG = C / 16;   // float4 groups per lane group
   constexpr int H = 16 * HB;
   constexpr int TP = TAN ? 16 : 32;  // pairs per tile
+  __shared__ v4u frags[L::kUnits];
   __shared__ __attribute__((aligned(16))) float lds[L::kFloats];
   __shared__ unsigned short lists[kPBWaves][kPBListN];
 
   // ---- stage the weights as A fragments (once per workgroup) ----
-  for (int f = threadIdx.x; f < 64 * C; f += blockDim.x) {
-    const int u = f & 3, lane = (f >> 2) & 63, rest = f >> 8;
-    const int sg = rest % CG, m = rest / CG;
-    const int k = (lane >> 4) * C4 + 4 * sg + u;
-    lds[L::kF1 + f] = p.w_in[k * kHid + 16 * m + (lane & 15)];
-  }
-  for (int f = threadIdx.x; f < 4096; f += blockDim.x) {
-    const int u = f & 3, lane = (f >> 2) & 63, kb = (f >> 8) & 3, m = f >> 10;
-    const int k = 16 * kb + 4 * (lane >> 4) + u, o = 16 * m + (lane & 15);
-    lds[L::kF2 + f] = p.w_1[k * kHid + o];
-    lds[L::kF3 + f] = p.w_2[k * kHid + o];
-  }
-  for (int f = threadIdx.x; f < 1024 * HB; f += blockDim.x) {
-    const int u = f & 3, lane = (f >> 2) & 63, kb = (f >> 8) & 3, m = f >> 10;
-    const int k = 16 * kb + 4 * (lane >> 4) + u;
-    lds[L::kF4 + f] = p.w_out[k * H + 16 * m + (lane & 15)];
-  }
+  const auto hidden_k = [](int step, int g, int j) { return 32 * step + 16 * (j >> 2) + 4 * g + (j & 3); };
+  stage_frags<C / 32, 4>(frags + L::kF1, [&](int k, int o) { return p.ln_w[k] * p.w_in[k * kHid + o]; },
+                         [](int step, int g, int j) { return g * C4 + 8 * step + j; });
+  stage_frags<2, 4>(frags + L::kF2, [&](int k, int o) { return p.w_1[k * kHid + o]; }, hidden_k);
+  stage_frags<2, 4>(frags + L::kF3, [&](int k, int o) { return p.gain * p.w_2[k * kHid + o]; }, hidden_k);
+  stage_frags<2, HB>(frags + L::kF4, [&](int k, int o) { return p.w_out[k * H + o]; }, hidden_k);
   for (int f = threadIdx.x; f < kHid; f += blockDim.x) {
     lds[L::kBin + f] = p.b_in[f];
     lds[L::kB1 + f] = p.b_1[f];
-    lds[L::kB2 + f] = p.b_2[f];
+    lds[L::kB2 + f] = p.gain * p.b_2[f];
   }
   for (int f = threadIdx.x; f < H; f += blockDim.x) lds[L::kBout + f] = p.b_out[f];
-  for (int f = threadIdx.x; f < C; f += blockDim.x) lds[L::kLnw + f] = p.ln_w[f];
   __syncthreads();
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -199,9 +225,9 @@ __global__ void __launch_bounds__(256, (pb_occupancy<C, HB>())) pair_bias_kernel
     const int64_t wstride = cmp ? p.e_blk * H : pair_stride * H;
     float* e_b = p.e + b * wstride;
     float* et_b = TAN ? p.e_t + b * wstride : nullptr;
+    const int64_t hstride = cmp ? p.e_blk : p.e_sh;  // between heads (uniform)
 
-    // The edge rows of the item's first tile; each tile then loads the next tile's rows as
-    // soon as its first layer has consumed its own, so the loads fly under layers 2-4.
+    // The edge rows of the item's first tile; each tile then loads the next tile's rows.
     int qi[2], qj[2], cpos[2];
     bool valid[2];
     float4 xin[2][CG];
@@ -211,34 +237,28 @@ __global__ void __launch_bounds__(256, (pb_occupancy<C, HB>())) pair_bias_kernel
     }
     for (int t = t0; t < t1; ++t) {
       // The weight fragments are the same for every tile; an offset the compiler cannot see
-      // through keeps their LDS reads inside the loop (hoisted, they would need 256 registers).
+      // through keeps their LDS reads inside the loop (hoisted, they would not fit the registers).
       int lz = 0;
       asm volatile("" : "+s"(lz));
       const float* W = lds + lz;
+      const v4u* F = frags + lz + lane;
 
-      // ---- layer 1: P = (x * w) W_in, with sum(x^2) and sum(x xdot) alongside ----
+      // ---- layer 1: P = x (w W_in), with sum(x^2) and sum(x xdot) alongside ----
       v4f acc[4][2];
 #pragma unroll
       for (int m = 0; m < 4; ++m) acc[m][0] = acc[m][1] = zero4();
       float s0 = 0.f, s1 = 0.f;  // sum x0^2; T = 1: sum x0 xdot, T = 0: sum x1^2
 #pragma unroll
-      for (int sg = 0; sg < CG; ++sg) {
-        const float4 w4 = lds4(W, L::kLnw + g * C4 + 4 * sg);
-        float4 a4[4];
+      for (int step = 0; step < C / 32; ++step) {
+        float x0[8], x1[8];
 #pragma unroll
-        for (int m = 0; m < 4; ++m) a4[m] = lds4(W, L::kF1 + ((m * CG + sg) * 64 + lane) * 4);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const float x0 = comp(xin[0][sg], u), x1 = comp(xin[1][sg], u), w = comp(w4, u);
-          s0 += x0 * x0;
-          s1 += TAN ? x0 * x1 : x1 * x1;
-          const float b0 = x0 * w, b1 = x1 * w;
-#pragma unroll
-          for (int m = 0; m < 4; ++m) {
-            acc[m][0] = mfma16x4(comp(a4[m], u), b0, acc[m][0]);
-            acc[m][1] = mfma16x4(comp(a4[m], u), b1, acc[m][1]);
-          }
+        for (int j = 0; j < 8; ++j) {
+          x0[j] = comp(xin[0][2 * step + (j >> 2)], j & 3);
+          x1[j] = comp(xin[1][2 * step + (j >> 2)], j & 3);
+          s0 += x0[j] * x0[j];
+          s1 += TAN ? x0[j] * x1[j] : x1[j] * x1[j];
         }
+        mm_step<4>(F + L::kF1 + step * 4 * L::kBlock, split8_clamped(x0), split8_clamped(x1), acc);
       }
       s0 += __shfl_xor(s0, 16);
       s0 += __shfl_xor(s0, 32);
@@ -248,110 +268,66 @@ __global__ void __launch_bounds__(256, (pb_occupancy<C, HB>())) pair_bias_kernel
       const float r0 = 1.0f / sqrtf(v0);
       // T = 1: the tangent's column scale rdot; T = 0: the second pair block's scale
       const float r1 = TAN ? (2.0f * s1 * inv_c) * (-0.5f * r0 / v0) : 1.0f / sqrtf(s1 * inv_c + p.eps);
+      // the next tile's rows, under the rest of this one
       int nqi[2] = {qi[0], qi[1]}, nqj[2] = {qj[0], qj[1]}, ncpos[2] = {cpos[0], cpos[1]};
       bool nvalid[2] = {false, false};
       if (t + 1 < t1) {
         tile_pairs<TAN>(t + 1, c, npairs, nk, rows_listed, keys_listed, list, nqi, nqj, nvalid, ncpos);
         load_rows<C, TAN>(edge_b, edge_tb, N, g, nqi, nqj, nvalid, xin);
       }
-      v4f h0[4][2];
+      v4f h[4][2];
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const float4 bi = lds4(W, L::kBin + 16 * m + 4 * g);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float P0 = acc[m][0][r], P1 = acc[m][1][r];
-          h0[m][0][r] = r0 * P0 + comp(bi, r);
-          h0[m][1][r] = TAN ? r0 * P1 + r1 * P0 : r1 * P1 + comp(bi, r);
+          h[m][0][r] = r0 * P0 + comp(bi, r);
+          h[m][1][r] = TAN ? r0 * P1 + r1 * P0 : r1 * P1 + comp(bi, r);
         }
       }
 
       // ---- layer 2: a = silu(h0 W_1 + b_1) (and its tangent) ----
 #pragma unroll
       for (int m = 0; m < 4; ++m) acc[m][0] = acc[m][1] = zero4();
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        float4 a4[4];
-#pragma unroll
-        for (int m = 0; m < 4; ++m) a4[m] = lds4(W, L::kF2 + ((m * 4 + kb) * 64 + lane) * 4);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int m = 0; m < 4; ++m) {
-            acc[m][0] = mfma16x4(comp(a4[m], u), h0[kb][0][u], acc[m][0]);
-            acc[m][1] = mfma16x4(comp(a4[m], u), h0[kb][1][u], acc[m][1]);
-          }
-      }
-      v4f act[4][2];
+      hidden_layer<4>(F + L::kF2, h, acc);
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const float4 b1 = lds4(W, L::kB1 + 16 * m + 4 * g);
+        const float4 b2 = lds4(W, L::kB2 + 16 * m + 4 * g);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float u0 = acc[m][0][r] + comp(b1, r);
           const float s = sigmoid(u0);
-          act[m][0][r] = u0 * s;
+          acc[m][0][r] = u0 * s;
           if (TAN) {
-            act[m][1][r] = acc[m][1][r] * (s + u0 * s * (1.0f - s));
+            acc[m][1][r] = acc[m][1][r] * (s + u0 * s * (1.0f - s));
           } else {
             const float u1 = acc[m][1][r] + comp(b1, r);
-            act[m][1][r] = u1 * sigmoid(u1);
+            acc[m][1][r] = u1 * sigmoid(u1);
           }
+          h[m][0][r] += comp(b2, r);
+          if (!TAN) h[m][1][r] += comp(b2, r);
         }
       }
 
-      // ---- layer 3: h1 = h0 + gain * (a W_2 + b_2) ----
-#pragma unroll
-      for (int m = 0; m < 4; ++m) acc[m][0] = acc[m][1] = zero4();
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        float4 a4[4];
-#pragma unroll
-        for (int m = 0; m < 4; ++m) a4[m] = lds4(W, L::kF3 + ((m * 4 + kb) * 64 + lane) * 4);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int m = 0; m < 4; ++m) {
-            acc[m][0] = mfma16x4(comp(a4[m], u), act[kb][0][u], acc[m][0]);
-            acc[m][1] = mfma16x4(comp(a4[m], u), act[kb][1][u], acc[m][1]);
-          }
-      }
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const float4 b2 = lds4(W, L::kB2 + 16 * m + 4 * g);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          h0[m][0][r] = h0[m][0][r] + p.gain * (acc[m][0][r] + comp(b2, r));
-          h0[m][1][r] = TAN ? h0[m][1][r] + p.gain * acc[m][1][r]
-                            : h0[m][1][r] + p.gain * (acc[m][1][r] + comp(b2, r));
-        }
-      }
+      // ---- layer 3: h1 = h0 + gain b_2 + a (gain W_2), summed straight into h ----
+      hidden_layer<4>(F + L::kF3, acc, h);
 
       // ---- layer 4: e = (h1 W_out + b_out) / div ----
       v4f o[HB][2];
 #pragma unroll
       for (int m = 0; m < HB; ++m) o[m][0] = o[m][1] = zero4();
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        float4 a4[HB];
-#pragma unroll
-        for (int m = 0; m < HB; ++m) a4[m] = lds4(W, L::kF4 + ((m * 4 + kb) * 64 + lane) * 4);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int m = 0; m < HB; ++m) {
-            o[m][0] = mfma16x4(comp(a4[m], u), h0[kb][0][u], o[m][0]);
-            o[m][1] = mfma16x4(comp(a4[m], u), h0[kb][1][u], o[m][1]);
-          }
-      }
+      hidden_layer<HB>(F + L::kF4, h, o);
 
       // ---- store: lane (g, c) holds heads 16 m + 4 g + r of its pair ----
 #pragma unroll
       for (int cb = 0; cb < 2; ++cb) {
         const int src = TAN ? 0 : cb;
         if (!valid[src]) continue;
-        float* const base = TAN && cb == 1 ? et_b : e_b;
-        float* dst = base + static_cast<int64_t>(qi[src]) * p.e_sq + static_cast<int64_t>(qj[src]) * p.e_sk;
+        const int64_t at = cmp ? cpos[src]  // the pair's compacted position in each head's block
+                               : static_cast<int64_t>(qi[src]) * p.e_sq + static_cast<int64_t>(qj[src]) * p.e_sk;
+        float* const dst = (TAN && cb == 1 ? et_b : e_b) + at + 4 * g * hstride;
         const bool with_bias = !(TAN && cb == 1);
 #pragma unroll
         for (int m = 0; m < HB; ++m) {
@@ -359,15 +335,11 @@ __global__ void __launch_bounds__(256, (pb_occupancy<C, HB>())) pair_bias_kernel
           float val[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) val[r] = (o[m][cb][r] + (with_bias ? comp(bo, r) : 0.0f)) * inv_div;
-          const int h = 16 * m + 4 * g;
-          if (cmp) {  // head h's block, the pair's compacted position
-#pragma unroll
-            for (int r = 0; r < 4; ++r) base[static_cast<int64_t>(h + r) * p.e_blk + cpos[src]] = val[r];
-          } else if (p.e_sh == 1) {
-            *reinterpret_cast<float4*>(dst + h) = make_float4(val[0], val[1], val[2], val[3]);
+          if (hstride == 1) {
+            *reinterpret_cast<float4*>(dst + 16 * m) = make_float4(val[0], val[1], val[2], val[3]);
           } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) dst[static_cast<int64_t>(h + r) * p.e_sh] = val[r];
+            for (int r = 0; r < 4; ++r) dst[(16 * m + r) * hstride] = val[r];
           }
         }
       }
@@ -384,12 +356,11 @@ __global__ void __launch_bounds__(256, (pb_occupancy<C, HB>())) pair_bias_kernel
 
 template <int C, int HB>
 hipError_t launch_pb(const PairBiasParams& p, bool tan, int64_t blocks, int cus, hipStream_t stream) {
-  const int64_t slots = static_cast<int64_t>(cus) * pb_occupancy<C, HB>();
-  const int grid = static_cast<int>(blocks < slots ? blocks : slots);
+  const int grid = static_cast<int>(blocks < cus ? blocks : cus);  // one workgroup per CU
   if (tan)
-    hipLaunchKernelGGL((pair_bias_kernel<C, HB, true>), dim3(grid), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((pair_bias_kernel<C, HB, true>), dim3(grid), dim3(64 * kPBWaves), 0, stream, p);
   else
-    hipLaunchKernelGGL((pair_bias_kernel<C, HB, false>), dim3(grid), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((pair_bias_kernel<C, HB, false>), dim3(grid), dim3(64 * kPBWaves), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -408,7 +379,7 @@ hipError_t launch_pb_c(const PairBiasParams& p, int H, bool tan, int64_t blocks,
 hipError_t launch_pair_bias(PairBiasParams p, int C, int H, bool tan, hipStream_t stream) {
   int cus = 0;
   if (hipError_t err = device_cu_count(&cus); err != hipSuccess) return err;
-  const int64_t waves = static_cast<int64_t>(cus) * 2 * kPBWaves;
+  const int64_t waves = static_cast<int64_t>(cus) * kPBWaves;
   // Parts per walker: about four items per wave, each part at least four tiles.
   const int64_t tp = tan ? 16 : 32;
   const int64_t tiles = (static_cast<int64_t>(p.N) * p.N + tp - 1) / tp;

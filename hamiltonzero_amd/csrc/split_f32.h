@@ -29,6 +29,12 @@ __device__ __forceinline__ v16f mfma32_bf16(bf16x8 a, bf16x8 b, v16f c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+// v_mfma_f32_16x16x32_bf16, lane l = 16 g + c: A[row c][k 8 g + j], B[k 8 g + j][col c], j = 0..7;
+// C/D as v_mfma_f32_16x16x4_f32.
+__device__ __forceinline__ v4f mfma16_bf16(bf16x8 a, bf16x8 b, v4f c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
 // Eight floats as three operands of eight bfloat16 each.
 struct Split8 {
   v4u h, m, l;
@@ -57,12 +63,58 @@ __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
   return s;
 }
 
+// The same for inputs that may lie above the largest bfloat16: finite values keep finite parts.
+__device__ __forceinline__ Split8 split8_clamped(const float (&x)[8]) {
+  constexpr float kMaxBf16 = 3.38953139e38f;
+  Split8 s;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float a = x[2 * j], b = x[2 * j + 1];
+    const uint32_t h = pack2_bf16(__builtin_amdgcn_fmed3f(a, -kMaxBf16, kMaxBf16),
+                                  __builtin_amdgcn_fmed3f(b, -kMaxBf16, kMaxBf16));
+    a -= __uint_as_float(h << 16);
+    b -= __uint_as_float(h & 0xffff0000u);
+    const uint32_t m = pack2_bf16(a, b);
+    a -= __uint_as_float(m << 16);
+    b -= __uint_as_float(m & 0xffff0000u);
+    s.h[j] = h;
+    s.m[j] = m;
+    s.l[j] = pack2_bf16(a, b);
+  }
+  return s;
+}
+
 __device__ __forceinline__ bf16x8 as_bf16x8(v4u u) { return __builtin_bit_cast(bf16x8, u); }
 
 // The six terms, smallest first: parts of a and of b (0 = h, 1 = m, 2 = l) of term t.
 constexpr int kSplitTerms = 6;
 constexpr int kSplitA[kSplitTerms] = {2, 0, 1, 1, 0, 0};
 constexpr int kSplitB[kSplitTerms] = {0, 2, 1, 0, 1, 0};
+
+// acc[m][cb] += A_m B_cb for MB row blocks and two column blocks, one K step of 32. W: this step's
+// A operands in LDS, [m][part][64 lanes], this lane's already added. Two row blocks at a time, so
+// four sums take turns on the matrix cores.
+template <int MB>
+__device__ __forceinline__ void mm_step(const v4u* W, const Split8& b0, const Split8& b1, v4f (&acc)[MB][2]) {
+  const bf16x8 b[2][3] = {{as_bf16x8(b0.h), as_bf16x8(b0.m), as_bf16x8(b0.l)},
+                          {as_bf16x8(b1.h), as_bf16x8(b1.m), as_bf16x8(b1.l)}};
+  constexpr int G = MB % 2 == 0 ? 2 : 1;
+#pragma unroll
+  for (int m0 = 0; m0 < MB; m0 += G) {
+    bf16x8 a[G][3];
+#pragma unroll
+    for (int i = 0; i < G; ++i)
+#pragma unroll
+      for (int part = 0; part < 3; ++part) a[i][part] = as_bf16x8(W[((m0 + i) * 3 + part) * 64]);
+#pragma unroll
+    for (int t = 0; t < kSplitTerms; ++t)
+#pragma unroll
+      for (int i = 0; i < G; ++i)
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb)
+          acc[m0 + i][cb] = mfma16_bf16(a[i][kSplitA[t]], b[cb][kSplitB[t]], acc[m0 + i][cb]);
+  }
+}
 
 __device__ __forceinline__ bool finite_f32(float x) {
   return (__float_as_uint(x) & 0x7f800000u) != 0x7f800000u;
