@@ -1,5 +1,5 @@
-// The MLP-class pair-bias producer on the float32 matrix cores (v_mfma_f32_16x16x4_f32): the
-// coupling bias of the tree's LevelEdgeAttn (src/hamiltonzero/model/tree.py:1392-1456), of the
+// The MLP-class pair-bias producer, float32 throughout (v_mfma_f32_16x16x4_f32; at hidden width 128
+// products as sums of bfloat16 ones): the coupling bias of the tree's LevelEdgeAttn (src/hamiltonzero/model/tree.py:1392-1456), of the
 // readout context (model/readout_leaf_context.py:694-712) and of the large-N sequence trunk
 // (evaluation/sequence_trunk.py:962-972, the tiled pair MLP). Per pair (i, j) of a walker, with
 // x = edge[b, i, j, :] (and, for the readout, one more input channel xe = extra[b, i, j]):
@@ -21,16 +21,17 @@
 // The residual gain is folded into W_2 and b_2, so the second product of a block accumulates
 // straight into h.
 //
-// At hidden width 128 the fp32 weights (W_in 96 x 128, W_1, W_2 128 x 128) exceed the LDS: W_1
-// and W_2 stay in LDS (128 KB) and W_in's fragments are read from memory (an L2-resident 48 KB
-// shared by every workgroup), one channel group ahead of the products. One such workgroup fits
-// a CU, and its four waves run one per SIMD with the whole register file (about 470 registers:
-// at two waves per SIMD the tile's h, activations and fragments spill 350-580 bytes per lane).
+// At hidden width 128 the weights exceed the LDS and pair_mlp_bias_wide_kernel passes them through it;
+// the float32 kernel serves that width only with 128 channels and 32 heads (W_1 and W_2 in LDS, 128
+// KB, W_in's fragments from memory one channel group ahead, one workgroup of four waves a CU).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "mhsea_device.h"
 #include "mhsea_launch.h"
+#include "split_f32.h"
 
 namespace hz {
 namespace {
@@ -425,6 +426,316 @@ __global__ void __launch_bounds__((64 * PMShape<C, KB, HB>::NW), (KB == 8 ? 1 : 
   }
 }
 
+// --------------------------------------------------------------------------------------
+// Hidden width 128
+// --------------------------------------------------------------------------------------
+// float32 products as six bfloat16 ones (split_f32.h, v_mfma_f32_16x16x32_bf16), the layers in
+// the same orientation: blocks 2s, 2s + 1 of a layer's result are the eight values per lane of the
+// next layer's B operand in K step s, slot j of lane group g feature 32 s + 16 (j / 4) + 4 g + j % 4.
+// The weights' three parts take 282 KB, so W_in and W_out stay in LDS and the K steps of W_1 and W_2
+// pass through it, two at a time (24 KB each): every thread reads eight weights of the next step
+// from memory (L2), splits them under this step's products and stores them, one barrier a step. The
+// eight waves (two a SIMD) each run their own tile of 16 pairs with tangent (32 without) in step,
+// so a staged step serves eight tiles; a workgroup's rounds cover an item's tiles eight at a time
+// and waves past its end only stage. 1024 walkers of 36 sites, C = 96, 16
+// heads, with tangent: 1310 us (2290 on the float32 matrix instruction), matrix cores 54% busy at
+// 1.92 GHz; what is left is the vector work of the splits and the wait for each round's rows.
+template <int C, int HB>
+struct PWShape {
+  static constexpr int KB = 8, HID = 128, H = 16 * HB, NW = 8, NT = 64 * NW;
+  static constexpr int kBlock = 3 * 64;                // 16-byte units of one (K step, M block)
+  static constexpr int kStep = KB * kBlock;            // one K step of W_1 or W_2
+  static constexpr int kWin = 0;                       // C / 32 steps x 8 blocks
+  static constexpr int kWout = kWin + C / 32 * kStep;  // 4 steps x HB blocks
+  static constexpr int kRing = kWout + 4 * HB * kBlock;
+  static constexpr int kUnits = kRing + 2 * kStep;
+  static constexpr int oBin = 0, oWe = HID, oB1 = 2 * HID, oB2 = 3 * HID, oNw = 4 * HID, oBout = 5 * HID,
+                       oSl = oBout + H;
+  static constexpr int kFloats = oSl + H;
+  static constexpr size_t kBytes = size_t(kUnits) * 16 + kFloats * 4 + kPMListN * 2 + 16;
+};
+
+template <int C, int HB, bool TAN>
+__global__ void __launch_bounds__((PWShape<C, HB>::NT), 2) pair_mlp_bias_wide_kernel(PairMlpParams p) {
+  using S = PWShape<C, HB>;
+  constexpr int KB = S::KB, HID = S::HID, H = S::H, CG = C / 16, C4 = C / 4, NW = S::NW;
+  constexpr int TP = TAN ? 16 : 32;  // pairs per tile
+  extern __shared__ v4u pw_smem[];
+  v4u* const frags = pw_smem;
+  float* const vecs = reinterpret_cast<float*>(pw_smem + S::kUnits);
+  unsigned short* const list = reinterpret_cast<unsigned short*>(vecs + S::kFloats);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, c = lane & 15;
+
+  // ---- W_in, W_out and the vectors (once per workgroup) ----
+  auto put = [](v4u* d, const Split8& sp) {
+    d[0] = sp.h;
+    d[64] = sp.m;
+    d[128] = sp.l;
+  };
+  for (int f = tid; f < C / 32 * KB * 64; f += S::NT) {
+    const int ln = f & 63, m = (f >> 6) % KB, step = (f >> 6) / KB;
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = p.w_in[((ln >> 4) * C4 + 8 * step + j) * HID + 16 * m + (ln & 15)];
+    put(frags + S::kWin + (step * KB + m) * S::kBlock + ln, split8(x));
+  }
+  for (int f = tid; f < 4 * HB * 64; f += S::NT) {
+    const int ln = f & 63, m = (f >> 6) % HB, step = (f >> 6) / HB;
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int k = 32 * step + 16 * (j >> 2) + 4 * (ln >> 4) + (j & 3);
+      x[j] = p.out_norm_w[k] * p.w_out[k * H + 16 * m + (ln & 15)];
+    }
+    put(frags + S::kWout + (step * HB + m) * S::kBlock + ln, split8(x));
+  }
+  for (int f = tid; f < HID; f += S::NT) {
+    vecs[S::oBin + f] = p.b_in[f];
+    vecs[S::oWe + f] = p.extra != nullptr ? p.w_in[C * HID + f] : 0.f;
+    vecs[S::oB1 + f] = p.b_1[f];
+    vecs[S::oB2 + f] = p.gain * p.b_2[f];
+    vecs[S::oNw + f] = p.norm_w[f];
+  }
+  for (int f = tid; f < H; f += S::NT) {
+    vecs[S::oBout + f] = p.b_out[f];
+    vecs[S::oSl + f] = p.slopes != nullptr ? p.slopes[f] : 0.f;
+  }
+  // This thread's weights of a step: M block `wave`, lane's column, eight k. Steps 0-3: diag(norm_w)
+  // W_1, 4-7: gain W_2; step s in ring slot s mod 2.
+  unsigned wo = 4 * (4 * g * HID + 16 * wave + c);  // bytes
+  float wr[8];
+  auto wload = [&](int step) {
+    asm volatile("" : "+v"(wo));  // as lz below: the addresses of eight steps would not fit
+    const float* const w = (step < 4 ? p.w_1 : p.w_2) + 32 * (step & 3) * HID;
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+      const float* const wj = w + 16 * jj * HID;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        wr[4 * jj + j] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(wj + j * HID) + wo);
+    }
+  };
+  auto wstore = [&](int step) {
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      x[j] = wr[j] * (step < 4 ? vecs[S::oNw + 32 * (step & 3) + 16 * (j >> 2) + 4 * g + (j & 3)] : p.gain);
+    put(frags + S::kRing + (step & 1) * S::kStep + wave * S::kBlock + lane, split8(x));
+  };
+
+  const int Nq = p.Nq, Nk = p.Nk;
+  const bool use_list = p.mask != nullptr && Nk <= kPMListN;
+  const float inv_hid = 1.0f / static_cast<float>(HID);
+  const float inv_div = 1.0f / p.div;
+  const bool alibi = p.slopes != nullptr;
+  wload(0);
+  __syncthreads();
+  wstore(0);
+  wload(1);
+
+  for (int64_t item = blockIdx.x; item < p.n_items; item += gridDim.x) {
+    const int64_t b = item / p.parts;
+    const int part = static_cast<int>(item - b * p.parts);
+    // ---- the walker's physical sites: every wave finds them, the first writes the list ----
+    int nk = Nk;
+    bool keys_listed = false, rows_listed = false;
+    __syncthreads();  // the last item's readers of the list are done
+    if (use_list) {
+      int n = 0;
+      for (int s0 = 0; s0 < Nk; s0 += 64) {
+        const int site = s0 + lane;
+        const bool phys = site < Nk && p.mask[b * Nk + site] != 0;
+        const uint64_t bal = __ballot(phys);
+        if (phys && wave == 0) list[n + __popcll(bal & ((1ull << lane) - 1ull))] = static_cast<unsigned short>(site);
+        n += __popcll(bal);
+      }
+      if (n > 0) {
+        nk = n;
+        keys_listed = true;
+        rows_listed = !p.key_mask;
+      } else if (!p.key_mask) {
+        continue;  // square mask, no physical site: the attention never reads this walker's bias
+      }
+    }
+    __syncthreads();
+    const int nrows = rows_listed ? nk : Nq;
+    const int npairs = nrows * nk;
+    const int ntiles = (npairs + TP - 1) / TP;
+    const int t0 = static_cast<int>(static_cast<int64_t>(ntiles) * part / p.parts);
+    const int t1 = static_cast<int>(static_cast<int64_t>(ntiles) * (part + 1) / p.parts);
+    float* e_b = p.e + b * static_cast<int64_t>(Nq) * Nk * H;
+    float* et_b = TAN ? p.e_t + b * static_cast<int64_t>(Nq) * Nk * H : nullptr;
+
+    for (int tb = t0; tb < t1; tb += NW) {
+      if (tb + wave >= t1) {  // no tile for this wave: its share of the weights and the barriers
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+          __syncthreads();
+          wstore((s + 1) & 7);
+          wload((s + 2) & 7);
+        }
+        continue;
+      }
+      // (loaded here: a round ahead they would not fit beside the layers' registers)
+      int qi[2], qj[2];
+      bool valid[2];
+      float4 xin[2][CG];
+      float xe[2];
+      pm_tile_pairs<TAN>(tb + wave, c, npairs, nk, rows_listed, keys_listed, list, qi, qj, valid);
+      pm_load_rows<C, TAN>(p, b, g, qi, qj, valid, xin, xe);
+      int lz = 0;
+      asm volatile("" : "+s"(lz));  // as in pair_mlp_bias_kernel: operand reads stay in the loop
+      const v4u* const F = frags + lz + lane;
+      const float* const W = vecs + lz;
+
+      // ---- in_proj: h = x W_in (+ xe w_e) + b_in ----
+      v4f h[KB][2];
+#pragma unroll
+      for (int m = 0; m < KB; ++m) h[m][0] = h[m][1] = zero4();
+#pragma unroll
+      for (int step = 0; step < C / 32; ++step) {
+        float x0[8], x1[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          x0[j] = cmp(xin[0][2 * step + (j >> 2)], j & 3);
+          x1[j] = cmp(xin[1][2 * step + (j >> 2)], j & 3);
+        }
+        mm_step<KB>(F + S::kWin + step * S::kStep, split8_clamped(x0), split8_clamped(x1), h);
+      }
+#pragma unroll
+      for (int m = 0; m < KB; ++m) {
+        const float4 bi = ld4(W, S::oBin + 16 * m + 4 * g);
+        const float4 we = ld4(W, S::oWe + 16 * m + 4 * g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          h[m][0][r] += fmaf(xe[0], cmp(we, r), cmp(bi, r));
+          h[m][1][r] += TAN ? xe[1] * cmp(we, r) : fmaf(xe[1], cmp(we, r), cmp(bi, r));
+        }
+      }
+
+      // ---- block: h += gain (silu(rms(h) W_1 + b_1) W_2 + b_2) ----
+      float r0, r1;
+      pm_rms<KB, TAN>(h, inv_hid, p.eps, r0, r1);
+      v4f a[KB][2];
+#pragma unroll
+      for (int m = 0; m < KB; ++m) a[m][0] = a[m][1] = zero4();
+      // One K step: the barrier makes ring slot s mod 2 readable and slot (s + 1) mod 2 free, where
+      // the next step's weights go after the products.
+      auto step_of = [&](auto s_c, const v4f (&x)[KB][2], v4f (&out)[KB][2]) {
+        constexpr int s = decltype(s_c)::value;
+        float x0[8], x1[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          x0[j] = x[2 * (s & 3) + (j >> 2)][0][j & 3];
+          x1[j] = x[2 * (s & 3) + (j >> 2)][1][j & 3];
+        }
+        const Split8 b0 = split8(x0), b1 = split8(x1);
+        __syncthreads();
+        mm_step<KB>(F + S::kRing + (s & 1) * S::kStep, b0, b1, out);
+        wstore((s + 1) & 7);
+        wload((s + 2) & 7);
+      };
+      using std::integral_constant;
+      step_of(integral_constant<int, 0>{}, h, a);
+      step_of(integral_constant<int, 1>{}, h, a);
+      step_of(integral_constant<int, 2>{}, h, a);
+      step_of(integral_constant<int, 3>{}, h, a);
+#pragma unroll
+      for (int m = 0; m < KB; ++m) {
+        const float4 b1 = ld4(W, S::oB1 + 16 * m + 4 * g);
+        const float4 b2 = ld4(W, S::oB2 + 16 * m + 4 * g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float P0 = a[m][0][r], P1 = a[m][1][r];
+          const float u0 = fmaf(r0, P0, cmp(b1, r));
+          const float sg = sigm(u0);
+          a[m][0][r] = u0 * sg;
+          if (TAN) {
+            a[m][1][r] = fmaf(r0, P1, r1 * P0) * (sg + u0 * sg * (1.0f - sg));
+          } else {
+            const float u1 = fmaf(r1, P1, cmp(b1, r));
+            a[m][1][r] = u1 * sigm(u1);
+          }
+          h[m][0][r] += cmp(b2, r);
+          if (!TAN) h[m][1][r] += cmp(b2, r);
+        }
+      }
+      step_of(integral_constant<int, 4>{}, a, h);
+      step_of(integral_constant<int, 5>{}, a, h);
+      step_of(integral_constant<int, 6>{}, a, h);
+      step_of(integral_constant<int, 7>{}, a, h);
+
+      // ---- out: e = (rms_out(h) W_out + b_out) / div - slope lca ----
+      float ro0, ro1;
+      pm_rms<KB, TAN>(h, inv_hid, p.eps, ro0, ro1);
+      v4f o[HB][2];
+#pragma unroll
+      for (int m = 0; m < HB; ++m) o[m][0] = o[m][1] = zero4();
+#pragma unroll
+      for (int step = 0; step < 4; ++step) {
+        float x0[8], x1[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          x0[j] = h[2 * step + (j >> 2)][0][j & 3];
+          x1[j] = h[2 * step + (j >> 2)][1][j & 3];
+        }
+        mm_step<HB>(F + S::kWout + step * HB * S::kBlock, split8(x0), split8(x1), o);
+      }
+      // ---- store: lane (g, c) holds heads 16 m + 4 g + r of its pair ----
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) {
+        const int src = TAN ? 0 : cb;
+        if (!valid[src]) continue;
+        float* dst = (TAN && cb == 1 ? et_b : e_b) + static_cast<int64_t>(qi[src]) * p.e_sq +
+                     static_cast<int64_t>(qj[src]) * p.e_sk + 4 * g * p.e_sh;
+        const bool tangent = TAN && cb == 1;
+        const float lvl = alibi && !tangent ? static_cast<float>(lca_level(p.row_offset + qi[src], qj[src])) : 0.f;
+#pragma unroll
+        for (int m = 0; m < HB; ++m) {
+          const float4 bo = ld4(W, S::oBout + 16 * m + 4 * g);
+          const float4 sl = ld4(W, S::oSl + 16 * m + 4 * g);
+          float val[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            if (tangent) {
+              val[r] = fmaf(ro0, o[m][1][r], ro1 * o[m][0][r]) * inv_div;
+            } else {
+              const float rr = (TAN || cb == 0) ? ro0 : ro1;
+              val[r] = fmaf(rr, o[m][cb][r], cmp(bo, r)) * inv_div - cmp(sl, r) * lvl;
+            }
+          }
+          if (p.e_sh == 1) {
+            *reinterpret_cast<float4*>(dst + 16 * m) = make_float4(val[0], val[1], val[2], val[3]);
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) dst[(16 * m + r) * p.e_sh] = val[r];
+          }
+        }
+      }
+    }
+  }
+}
+
+template <int C, int HB>
+hipError_t launch_pw(PairMlpParams p, bool tan, int cus, hipStream_t stream) {
+  using S = PWShape<C, HB>;
+  // Parts per walker: four items per CU, each at least two rounds of eight tiles.
+  const int64_t tiles = (static_cast<int64_t>(p.Nq) * p.Nk + (tan ? 16 : 32) - 1) / (tan ? 16 : 32);
+  int64_t parts = (4 * static_cast<int64_t>(cus) + p.B - 1) / p.B;
+  parts = parts > tiles / (2 * S::NW) ? tiles / (2 * S::NW) : parts;
+  parts = parts < 1 ? 1 : (parts > (1 << 20) ? (1 << 20) : parts);
+  p.parts = static_cast<int>(parts);
+  p.n_items = p.B * parts;
+  auto kern = tan ? pair_mlp_bias_wide_kernel<C, HB, true> : pair_mlp_bias_wide_kernel<C, HB, false>;
+  hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(S::kBytes));
+  if (err != hipSuccess) return err;
+  const int grid = static_cast<int>(p.n_items < cus ? p.n_items : cus);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(S::NT), S::kBytes, stream, p);
+  return hipGetLastError();
+}
+
 template <int C, int KB, int HB>
 hipError_t launch_pm(const PairMlpParams& p, bool tan, int cus, hipStream_t stream) {
   using S = PMShape<C, KB, HB>;
@@ -450,12 +761,26 @@ hipError_t launch_pm_h(const PairMlpParams& p, int H, bool tan, int cus, hipStre
   }
 }
 
+// Hidden width 128: the kernel above while its weights fit the LDS (every shape but 128 channels with
+// 32 heads, 174 KB), else the float32 one.
+template <int C>
+hipError_t launch_pm_wide(const PairMlpParams& p, int H, bool tan, int cus, hipStream_t stream) {
+  constexpr size_t kLds = 160 * 1024;
+  static_assert(PWShape<C, 1>::kBytes <= kLds, "one head block fits at every channel count");
+  if (H == 16) return launch_pw<C, 1>(p, tan, cus, stream);
+  if (H != 32) return hipErrorInvalidValue;
+  if constexpr (PWShape<C, 2>::kBytes <= kLds)
+    return launch_pw<C, 2>(p, tan, cus, stream);
+  else
+    return launch_pm<C, 8, 2>(p, tan, cus, stream);
+}
+
 template <int C>
 hipError_t launch_pm_c(const PairMlpParams& p, int hidden, int H, bool tan, int cus, hipStream_t stream) {
   switch (hidden) {
     case 32: return launch_pm_h<C, 2>(p, H, tan, cus, stream);
     case 64: return launch_pm_h<C, 4>(p, H, tan, cus, stream);
-    case 128: return launch_pm_h<C, 8>(p, H, tan, cus, stream);
+    case 128: return launch_pm_wide<C>(p, H, tan, cus, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -108,6 +108,24 @@ def test_pair_mlp_bias_matches_oracle(case):
         assert rel(to_ref(e_t.cpu().numpy())[read], want_t[read]) <= TOL, "e_t"
 
 
+@pytest.mark.parametrize(
+    "B,N,C,H,T,mask_kind,layout",
+    [
+        (1, 1, 32, 16, 1, "none", "qkh"),            # one pair: one wave of a round's eight has a tile
+        (3, 12, 64, 32, 1, "none", "qhk"),           # nine tiles: a second round of one
+        (2, 16, 96, 16, 0, "none", "qkh"),           # eight tiles of 32 pairs exactly
+        (5, 17, 128, 16, 1, "square_empty", "qkh"),  # the most LDS; a walker without sites before others
+        (300, 6, 96, 32, 1, "square_empty", "qkh"),  # more items than CUs
+        (2, 9, 128, 32, 1, "key_empty", "qhk"),      # weights past the LDS: the float32 kernel
+    ],
+)
+def test_pair_mlp_bias_hidden_128_rounds(B, N, C, H, T, mask_kind, layout):
+    """Hidden width 128, eight tiles a round in step: partial and single-tile rounds, walkers
+    skipped between others, every channel count's LDS layout."""
+    test_pair_mlp_bias_matches_oracle((f"rounds_{B}_{N}_{C}_{H}", B, N, N, C, 128, H, 1, T, False, True, 3, mask_kind,
+                                       layout))
+
+
 def test_pair_mlp_bias_feeds_the_gated_rect_attention():
     """The large-N chain (sequence_trunk.py:962-984): the producer's bias with a global row
     offset, then the gated rectangular attention, against the oracle's chain."""
