@@ -325,6 +325,20 @@ def mhsea_fwd_jvp_gated(
     return y, (None if ty is None else (ty if batched else ty[0]))
 
 
+def gate_collapse(out: Tensor) -> Tensor:
+    """``y = sigmoid(out[:, :, :H/2]) * out[:, :, H/2:]`` of a kept attention output ``out [B, N,
+    H, D]`` (``hz_gate_collapse_fwd``; float32, H even)."""
+    if out.dim() != 4 or out.dtype != torch.float32 or not out.is_cuda:
+        raise ValueError("out must be a float32 GPU tensor [B, N, H, D]")
+    B, N, H, D = out.shape
+    if H % 2:
+        raise ValueError(f"the gated collapse pairs head h with h + H/2: H must be even, got {H}")
+    out = out.contiguous()
+    y = torch.empty((B, N, H // 2, D), dtype=out.dtype, device=out.device)
+    _native.check(_native.lib().hz_gate_collapse_fwd(_stream(out.device), _ptr(out), _ptr(y), B, N, H, D))
+    return y
+
+
 def gated_out_proj(y: Tensor, w_o: Tensor, ty: Optional[Tensor] = None,
                    mask: Optional[Tensor] = None) -> Tuple[Tensor, Optional[Tensor]]:
     """The attention block's output projection after the gate collapse: ``delta = y_flat @

@@ -169,10 +169,53 @@ class _GatedAD(torch.autograd.Function):
         return torch.zeros_like(y) if ty is None else ty
 
 
+class _GatedTrainAD(torch.autograd.Function):
+    """(y, out, lse) of the same call where a gradient is wanted: the attention's (out, lse) are
+    kept for reverse mode and y is the collapse of out, so the backward pass needs no second
+    forward (a [1024, 64, 32, 16] call with bias and its gradients: 832 -> 759 us)."""
+
+    @staticmethod
+    def forward(q, k, e, v, mask, opts):
+        scale, key_mask, e_layout = opts
+        out, lse = kernels.mhsea_fwd(q, k, v, mask, e, scale=scale, key_mask=key_mask, e_layout=e_layout)
+        return kernels.gate_collapse(out), out, lse
+
+    @staticmethod
+    def setup_context(ctx, inputs, output):
+        q, k, e, v, mask, opts = inputs
+        _y, out, lse = output
+        ctx.opts = opts
+        ctx.mark_non_differentiable(out, lse)
+        ctx.save_for_backward(q, k, e, v, mask, out, lse)
+        ctx.save_for_forward(q, k, e, v, mask)
+
+    @staticmethod
+    def backward(ctx, dy, _dout, _dlse):
+        q, k, e, v, mask, out, lse = ctx.saved_tensors
+        scale, key_mask, e_layout = ctx.opts
+        dq, dk, de, dv = kernels.mhsea_bwd_gated(
+            q, k, v, mask, lse, out, dy.contiguous(), e,
+            want_de=bool(ctx.needs_input_grad[2]), scale=scale, key_mask=key_mask, e_layout=e_layout,
+        )
+        return dq, dk, de, dv, None, None
+
+    @staticmethod
+    def jvp(ctx, qt, kt, et, vt, _mask_t, _opts_t):
+        q, k, e, v, mask = ctx.saved_tensors[:5]
+        scale, key_mask, e_layout = ctx.opts
+        y, ty = kernels.mhsea_fwd_jvp_gated(q, k, v, mask, qt, kt, vt, e=e, et=et, scale=scale, key_mask=key_mask,
+                                            e_layout=e_layout)
+        return (torch.zeros_like(y) if ty is None else ty), None, None
+
+
 def gated_edge_attention(q, k, e, v, mask, *, scale: float = 1.0, key_mask: bool = False, e_layout: str = "qhk"):
     """Differentiable head-collapsed attention ``sigmoid(gate) * value`` (trunk.py:130-137 for
     the tuned path): ``[B, N, H, D]`` operands with H = 2 * n_heads, result ``[B, N, H/2, D]``.
     Serves what ``hz_mhsea_fwd_jvp_gated`` serves (fp32, any N and head dimension, even H)."""
+    wants_grad = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (q, k, e, v))
+    # the compacted bias layout has no reverse mode, and H odd or another dtype is refused there
+    if wants_grad and e_layout != "compact" and q.dtype == torch.float32 and q.dim() == 4 and q.shape[2] % 2 == 0:
+        return _GatedTrainAD.apply(q, k, e, v, mask, (float(scale), bool(key_mask), e_layout))[0]
     return _GatedAD.apply(q, k, e, v, mask, (float(scale), bool(key_mask), e_layout))
 
 

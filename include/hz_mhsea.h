@@ -209,6 +209,14 @@ int hz_mhsea_bwd(hipStream_t stream,
                  int dtype, float scale, int flags);
 
 /*
+ * The head collapse alone (trunk.py:134-137), y = sigmoid(out[:, :, :H/2]) * out[:, :, H/2:], of
+ * an attention output out [B, N, H, D] that the caller keeps: hz_mhsea_fwd then this gives
+ * hz_mhsea_bwd_gated its (out, lse) without a second forward, where hz_mhsea_fwd_jvp_gated
+ * (which never writes out) needs one. float32; H even; y [B, N, H/2, D].
+ */
+int hz_gate_collapse_fwd(hipStream_t stream, const float* out, float* y, int64_t B, int64_t N, int64_t H, int64_t D);
+
+/*
  * Reverse mode of the gated head collapse (hz_mhsea_fwd_jvp_gated's y = sigmoid(g) v):
  * cotangents of (q, k, e, v) for the cotangent dy [B, N, H/2, D] of y. Replaces the reverse
  * pass JAX derives for the trunk's attention call followed by trunk.py:134-137 (the

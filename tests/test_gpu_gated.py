@@ -122,7 +122,7 @@ def test_gated_equals_unfused_composition_at_c2_shape():
 
 @pytest.mark.parametrize("with_e", [False, True])
 def test_gated_edge_attention_autograd(with_e):
-    """``gated_edge_attention``: reverse mode (recomputed out, lse; attention backward on the
+    """``gated_edge_attention``: reverse mode (kept out, lse; attention backward on the
     collapse's cotangent) against the float64 oracle's VJP of the composite, and forward mode
     (the fused kernel's tangent) against ``gated_fwd_jvp``."""
     import torch.autograd.forward_ad as fwAD
@@ -157,6 +157,36 @@ def test_gated_edge_attention_autograd(with_e):
         torch.cuda.synchronize()
         _, want_t = O.gated_fwd_jvp(q, k, e, v, mask, tq[0], tk[0], te[0] if with_e else None, tv[0], scale=scale)
         assert rel(ty.cpu().numpy(), want_t) <= TOL
+
+
+@pytest.mark.parametrize("B,N,H,D,key_mask,layout", [(1, 1, 2, 8, False, "qhk"), (5, 33, 4, 16, False, "qkh"),
+                                                     (2, 70, 2, 64, False, "qhk"), (3, 24, 6, 32, True, "qhk")])
+def test_gated_edge_attention_keeps_out_and_lse(B, N, H, D, key_mask, layout):
+    """Where a gradient is wanted the collapse runs on the kept attention output: the same y as the
+    fused kernel (both round sigmoid and product once; attention sums differ between the kernel
+    families, TOL) and the gradients of hz_mhsea_bwd_gated on (out, lse) bit for bit, walkers
+    without a physical site included."""
+    from hamiltonzero_amd import gated_edge_attention, kernels
+
+    _say(f"gated kept out {(B, N, H, D, key_mask, layout)}")
+    gen = torch.Generator(device="cuda").manual_seed(B * N + H)
+    rnd = lambda *s: torch.randn(s, generator=gen, device="cuda")  # noqa: E731
+    q, k, v = (rnd(B, N, H, D) for _ in range(3))
+    e = 0.5 * rnd(*kernels.e_shape(B, N, H, layout))
+    mask = torch.rand((B, N), generator=gen, device="cuda") < 0.7
+    mask[0] = B == 1
+    dy = rnd(B, N, H // 2, D)
+    opts = dict(scale=D ** -0.5, key_mask=key_mask, e_layout=layout)
+    with torch.no_grad():
+        fused = gated_edge_attention(q, k, e, v, mask, **opts)
+    leaves = [x.clone().requires_grad_(True) for x in (q, k, e, v)]
+    y = gated_edge_attention(leaves[0], leaves[1], leaves[2], leaves[3], mask, **opts)
+    assert rel(y.detach().cpu().numpy(), fused.cpu().numpy()) <= TOL
+    got = torch.autograd.grad(y, leaves, dy)
+    out, lse = kernels.mhsea_fwd(q, k, v, mask, e, **opts)
+    want = kernels.mhsea_bwd_gated(q, k, v, mask, lse, out, dy, e, **opts)
+    for a, b in zip(got, (want[0], want[1], want[2], want[3])):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("T,masked,shape", [(0, False, (3, 17, 2, 8, 5)), (1, True, (64, 64, 16, 16, 512)),
