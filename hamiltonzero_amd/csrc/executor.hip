@@ -876,13 +876,13 @@ __global__ void __launch_bounds__(256) leaf_pair_level_kernel(const float* __res
   }
 }
 
-// Whether the basis serves: at least one pair, inputs that fit its one K step, and no more basis
+// Whether the basis serves: at least one pair (and no more than a grid's second dimension), inputs that fit its one K step, and no more basis
 // rows than walker rows, neither at the leaves (2 nq: the basis is held in half a leaf buffer) nor
 // at the pairs (nq^2). At that line (16 walkers, nq = 4, fine-tune widths) the whole wavefunction
 // takes 948 -> 732 us at 64 sites and 660 -> 456 us at 8; 500 x 64 sites 4618 -> 1978 us, 1024 x 64
 // 8799 -> 3386 us.
 bool basis_serves(int64_t B, int n, int nq) {
-  return n > 1 && nq <= kMaxBasis && B >= static_cast<int64_t>(nq) * nq && B >= 2 * nq;
+  return n > 1 && n / 2 <= 65535 && nq <= kMaxBasis && B >= static_cast<int64_t>(nq) * nq && B >= 2 * nq;
 }
 
 hipError_t launch_merge(const float* T, const float* ua, const float* ub, float* out, int64_t M, int G,

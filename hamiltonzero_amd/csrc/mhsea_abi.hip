@@ -514,7 +514,7 @@ int hz_quadrilinear_merge(hipStream_t stream, const float* T, const float* u_a, 
   if (R != 32) return fail(HZ_EINVAL, "the merge rank R must be 32, got %lld", (long long)R);
   if (M < 1 || G < 1) return fail(HZ_EINVAL, "M and G must be >= 1, got M=%lld G=%lld", (long long)M, (long long)G);
   if (G > 65535) return fail(HZ_EINVAL, "G = %lld exceeds the grid limit", (long long)G);
-  if ((M + 255) / 256 > 0x7fffffffLL) return fail(HZ_EINVAL, "M = %lld exceeds the grid limit", (long long)M);
+  if ((M + 127) / 128 > 0x7fffffffLL) return fail(HZ_EINVAL, "M = %lld exceeds the grid limit", (long long)M);
   HZ_REQUIRE(T);
   HZ_REQUIRE(u_a);
   HZ_REQUIRE(u_b);
@@ -576,7 +576,10 @@ int hz_pair_bias(hipStream_t stream, const float* edge, const float* edge_t, con
   if (hidden != 64) return fail(HZ_EINVAL, "hidden = %lld: the bias MLP's hidden width must be 64", (long long)hidden);
   if (H != 16 && H != 32 && H != 64) return fail(HZ_EINVAL, "H = %lld: heads must be 16, 32 or 64", (long long)H);
   if (T != 0 && T != 1) return fail(HZ_EINVAL, "T = %lld: T must be 0 or 1", (long long)T);
-  if (flags & ~(HZ_FLAG_KEY_MASK | HZ_FLAG_E_QKH | HZ_FLAG_E_COMPACT)) return fail(HZ_EINVAL, "unknown flag bits 0x%x", flags);
+  if (flags & ~(HZ_FLAG_KEY_MASK | HZ_FLAG_E_QKH | HZ_FLAG_E_COMPACT | HZ_FLAG_E_ZERO))
+    return fail(HZ_EINVAL, "unknown flag bits 0x%x", flags);
+  if ((flags & HZ_FLAG_E_ZERO) && !((flags & HZ_FLAG_E_COMPACT) && mask != nullptr))
+    return fail(HZ_EINVAL, "HZ_FLAG_E_ZERO needs HZ_FLAG_E_COMPACT and a mask");
   if ((flags & HZ_FLAG_E_COMPACT) && (flags & (HZ_FLAG_KEY_MASK | HZ_FLAG_E_QKH)))
     return fail(HZ_EINVAL, "HZ_FLAG_E_COMPACT excludes HZ_FLAG_KEY_MASK and HZ_FLAG_E_QKH");
   if ((flags & HZ_FLAG_E_COMPACT) && mask != nullptr && N > 256)
@@ -617,6 +620,7 @@ int hz_pair_bias(hipStream_t stream, const float* edge, const float* edge_t, con
   p.B = B;
   p.N = static_cast<int>(N);
   set_e_strides(N, H, flags, p.e_sq, p.e_sh, p.e_sk);
+  p.zero_rest = (flags & HZ_FLAG_E_ZERO) != 0;
   if (flags & HZ_FLAG_E_COMPACT) p.e_blk = N * ((N + 3) & ~int64_t(3));
   p.gain = inner_gain;
   p.eps = eps;
@@ -648,7 +652,7 @@ int hz_compiled_wavefunction(hipStream_t stream, const float* q, const float* q_
   if (n_sites > 0x7fffffffLL || d_q > 0x7fffffffLL || d_z > 0x7fffffffLL || R_leaf > 0x7fffffffLL ||
       R_merge > 0x7fffffffLL || R_out > 0x7fffffffLL)
     return fail(HZ_EINVAL, "dimensions exceed the 32-bit range");
-  if ((B * n_sites + 127) / 128 > 65535 || (B * n_sites + 255) / 256 > 0x7fffffffLL)
+  if ((B * n_sites + 127) / 128 > 65535 || (B * n_sites + 127) / 128 > 0x7fffffffLL)
     return fail(HZ_EINVAL, "B * n_sites = %lld exceeds the grid limit", (long long)(B * n_sites));
   if (!std::isfinite(merge_eps) || merge_eps < 0.0f) return fail(HZ_EINVAL, "merge_eps must be finite and >= 0");
   const int64_t need = hz::compiled_wavefunction_workspace_bytes(B, n_sites, d_z, R_leaf, d_m, R_merge, R_out);

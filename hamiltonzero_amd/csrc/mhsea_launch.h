@@ -190,6 +190,7 @@ struct PairBiasParams {
   int64_t B;
   int N;
   int64_t e_sq, e_sh, e_sk;
+  int zero_rest;        // compacted layout with a mask: the entries no pair fills are zeroed
   int64_t e_blk;        // > 0: compacted layout, floats per (walker, head) block (N * ceil4(N))
   float gain, eps, div;
   bool key_mask;        // compute every query row (key-mask attention semantics)

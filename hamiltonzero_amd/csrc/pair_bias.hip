@@ -205,6 +205,18 @@ __global__ void __launch_bounds__(64 * kPBWaves, 2) pair_bias_kernel(PairBiasPar
         n += __popcll(bal);
       }
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      // The entries of the walker's compacted blocks that no pair fills (the pad of each row, the
+      // tail), zeroed while the matrix cores work: heads part, part + parts, ... of this item.
+      if (p.zero_rest) {
+        const int n4 = (n + 3) & ~3;
+        for (int h = part; h < H; h += p.parts)
+          for (int t = 0; t < (TAN ? 2 : 1); ++t) {
+            float* const blk = (t == 0 ? p.e : p.e_t) + (b * H + h) * p.e_blk;
+            for (int i = n * n4 + 4 * lane; i < p.e_blk; i += 256) *reinterpret_cast<v4f*>(blk + i) = zero4();
+            for (int i = lane; i < n; i += 64)
+              for (int j = n; j < n4; ++j) blk[i * n4 + j] = 0.f;
+          }
+      }
       if (n > 0) {
         nk = n;
         keys_listed = true;

@@ -132,9 +132,9 @@ class _MhseaAD(torch.autograd.Function):
 class _GatedAD(torch.autograd.Function):
     """y = sigmoid(out[:, :, :H/2]) * out[:, :, H/2:] of MHSEA(q, k, e, v, mask), the trunk's
     head collapse (trunk.py:134-137). The forward and forward mode run the fused kernel
-    (``hz_mhsea_fwd_jvp_gated``); reverse mode recomputes (out, lse) and runs
-    ``hz_mhsea_bwd_gated`` (the collapse's cotangent formed on the GPU, then the attention
-    backward)."""
+    (``hz_mhsea_fwd_jvp_gated``); the calls that want a gradient run :class:`_GatedTrainAD`, so this
+    reverse mode (recomputing (out, lse) for ``hz_mhsea_bwd_gated``) serves only those it leaves
+    here, which the C entry then answers or refuses."""
 
     @staticmethod
     def forward(q, k, e, v, mask, opts):

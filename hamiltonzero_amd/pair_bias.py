@@ -100,11 +100,13 @@ def coupling_bias(
         tangents = edge_t.unsqueeze(0) if single else edge_t
         tangents = _check("edge_t", tangents, dev, (tangents.shape[0], B, N, N, C))
     eshape = kernels.e_shape(B, N, H, e_layout)
-    alloc = torch.zeros if m is not None else torch.empty
+    # the compacted layout's producer zeroes what no pair fills itself, under its products
+    zero = m is not None and e_layout == "compact"
+    alloc = torch.zeros if m is not None and not zero else torch.empty
     e = alloc(eshape, dtype=torch.float32, device=dev)
     T = 0 if tangents is None else tangents.shape[0]
     e_t = alloc((T, *eshape), dtype=torch.float32, device=dev) if T else None
-    flags = kernels._flags(key_mask, e_layout)
+    flags = kernels._flags(key_mask, e_layout) | (_native.HZ_FLAG_E_ZERO if zero else 0)
     lib = _native.lib()
     stream = torch.cuda.current_stream(dev).cuda_stream
     div = float(torch.sqrt(torch.tensor(float(d_head), dtype=torch.float32)))  # jnp.sqrt in float32

@@ -89,7 +89,8 @@ enum hz_flags {
      HZ_FLAG_KEY_MASK), float32, and only where the N <= 64 producer/consumer kernel serves
      the shape (N <= 64, D in {8, 16, 32}); accepted by hz_mhsea_fwd, hz_mhsea_jvp,
      hz_mhsea_fwd_jvp and hz_mhsea_fwd_jvp_gated, refused (HZ_EINVAL) elsewhere. */
-  HZ_FLAG_E_COMPACT = 8
+  HZ_FLAG_E_COMPACT = 8,
+  HZ_FLAG_E_ZERO = 16 /* hz_pair_bias with HZ_FLAG_E_COMPACT: every entry no pair fills is zeroed */
 };
 
 enum hz_status {

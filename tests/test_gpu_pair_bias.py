@@ -260,3 +260,29 @@ def test_attention_never_reads_uncomputed_bias(route):
     clean, poisoned = run(0.0), run(float("nan"))
     for a, b in zip(clean, poisoned):
         assert np.array_equal(a, b, equal_nan=False), name
+
+
+@pytest.mark.parametrize("B,N,H,T", [(3, 7, 16, 1), (2, 64, 32, 1), (4, 33, 64, 0), (70, 18, 32, 1), (2, 130, 16, 0)])
+def test_compact_output_is_zero_where_no_pair_lies(B, N, H, T):
+    """coupling_bias in the compacted layout into memory that held NaN: the pairs of the plain layout
+    (bit for bit) and zeros everywhere else - row pads, tails, walkers with no or one site."""
+    from hamiltonzero_amd import kernels, pair_bias
+
+    print(f"[case] compact zeros B={B} N={N} H={H} T={T}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(B + N)
+    rnd = lambda *s: torch.randn(s, generator=gen, device="cuda")  # noqa: E731
+    C, hid = 32, 64
+    params = {"ln_w": 1 + 0.1 * rnd(C), "w_in": rnd(C, hid) / 6, "b_in": rnd(hid), "w_1": rnd(hid, hid) / 8,
+              "b_1": rnd(hid), "w_2": rnd(hid, hid) / 8, "b_2": rnd(hid), "w_out": rnd(hid, H) / 8, "b_out": rnd(H)}
+    mask = torch.rand((B, N), generator=gen, device="cuda") < 0.6
+    mask[0] = False
+    mask[1] = False
+    mask[1, N // 2] = True
+    edge, edge_t = rnd(B, N, N, C), (rnd(B, N, N, C) if T else None)
+    opts = dict(d_head=16, inner_gain=0.5, mask=mask, edge_t=edge_t)
+    plain = pair_bias.coupling_bias(edge, params, **opts)
+    dirty = [torch.full(kernels.e_shape(B, N, H, "compact"), float("nan"), device="cuda") for _ in range(1 + T)]
+    del dirty  # the caching allocator hands this memory out again
+    got = pair_bias.coupling_bias(edge, params, e_layout="compact", **opts)
+    for a, b in zip(got if T else (got,), plain if T else (plain,)):
+        assert torch.equal(a, kernels.compact_bias(b, mask))
