@@ -179,12 +179,6 @@ quadrilinear_merge_kernel(const float* __restrict__ T, const float* __restrict__
 // Tiled GEMM with epilogues
 // --------------------------------------------------------------------------------------
 constexpr int kBM = 128, kBN = 128, kBK = 16;
-// Row lengths of gemm_rows_f32_kernel's As[k][row] and Bs[k][col] (floats): 16 more than a tile,
-// so the four k rows of one operand read (lanes 16 g + c read row g, column c) fall on distinct
-// banks. A's transposed stores put column r of k rows 4q .. 4q + 3 at r ^ 16 q, so the four lanes
-// that share r (q = 0..3, rows 4 x 144 floats apart, one bank) write four banks; a read's four
-// rows share q, so it still covers one aligned 16-column block per row.
-constexpr int kBPad = kBN + 16;
 
 constexpr int kAhead = 2;  // K slices in flight in registers (even)
 
@@ -363,15 +357,23 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ Bm, float
 // are compacted into the LDS tile, so only ceil(n / 16) row blocks are multiplied, and its
 // masked rows of C are written as zeros. Wave w owns columns [32 w, 32 w + 32) of the tile for
 // every row block. Workgroups are numbered so that the column tiles of one row block run on
-// one XCD (one L2 holds their A rows). K and N are multiples of 4 (16-byte staging loads).
+// one XCD (one L2 holds their A rows). K and N are multiples of 4 (16-byte loads of A, stores of
+// zeros). float32 products as six bfloat16 ones (split_f32.h): the slice's rows are split once, by
+// all threads, into 48 KB of LDS that every wave reads; a wave's columns of B come from memory to its
+// registers and are split there, a slice ahead of their products. Two workgroups of 50 KB and 244
+// registers a CU, so one stages under the other's products. Bound by memory (its output alone is
+// 134 MB) and the splits: 65536 rows, 36 of 64 physical, 256 x 512, y and its tangent 210 -> 151 us
+// (the float32 matrix instruction was 53% busy).
 constexpr int kRM = 256;  // 16 row blocks: the dispatch below instantiates 1..16
-constexpr int kRMPad = kRM + 16;
+constexpr int kRK = 32;   // K per slice: one matrix step
 
 __global__ void __launch_bounds__(256, 2)
 gemm_rows_f32_kernel(const float* __restrict__ A, const float* __restrict__ Bm, float* __restrict__ C,
                      const uint8_t* __restrict__ mask, int64_t M, int N, int K, int ncol) {
-  __shared__ float As[2][kBK][kRMPad];
-  __shared__ float Bs[2][kBK][kBPad];
+  // a slice of A as ready operands, [row block][part][64 lanes]: slot s's chunk of lane group g at
+  // lane 16 g + (s mod 16 ^ 2 g), which spreads any 8 consecutive lanes of a store or a read over
+  // the banks
+  __shared__ v4u As[kRM / 16 * 3 * 64];
   __shared__ int16_t prow[kRM], mrow[kRM];
   __shared__ int counts[8];
   const int tid = threadIdx.x;
@@ -417,79 +419,70 @@ gemm_rows_f32_kernel(const float* __restrict__ A, const float* __restrict__ Bm, 
   }
   if (n == 0) return;  // workgroup-uniform
 
-  // global -> register staging: A slots 256 x 16 as 1024 float4 (slot = it / 4, k4 = it % 4;
-  // slots past n stay zero; each slot's row offset is fixed for the whole K loop), B tile
-  // 16 x 128 as 512 float4 (k = it / 32, n4 = it % 32)
-  int64_t aoff[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int slot = (tid + 256 * u) >> 2;
-    aoff[u] = slot < n ? (m0 + prow[slot]) * K : -1;
-  }
-  float4 ra[4], rb[2];
-  auto gload = [&](int k0) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int kk = k0 + 4 * ((tid + 256 * u) & 3);
-      ra[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (aoff[u] >= 0 && kk < K) ra[u] = *reinterpret_cast<const float4*>(A + aoff[u] + kk);
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int it = tid + 256 * u;
-      const int kb = k0 + (it >> 5);
-      const int nn = n0 + 4 * (it & 31);
-      rb[u] = (kb < K && nn < N) ? *reinterpret_cast<const float4*>(Bm + static_cast<int64_t>(kb) * N + nn)
-                                 : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-  };
-  auto sstore = [&](int buf) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int it = tid + 256 * u;
-      const int r = it >> 2, k4 = 4 * (it & 3);
-      const int rs = r ^ (16 * ((k4 >> 2) & 3));  // as in gemm_f32_kernel
-      As[buf][k4 + 0][rs] = ra[u].x;
-      As[buf][k4 + 1][rs] = ra[u].y;
-      As[buf][k4 + 2][rs] = ra[u].z;
-      As[buf][k4 + 3][rs] = ra[u].w;
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int it = tid + 256 * u;
-      *reinterpret_cast<float4*>(&Bs[buf][it >> 5][4 * (it & 31)]) = rb[u];
-    }
-  };
-
   // the K loop and the stores for NMT = ceil(n / 16) row blocks, a compile-time count so
   // the products run without branches
   auto body = [&](auto nmt_c) {
     constexpr int NMT = decltype(nmt_c)::value;
+    constexpr int NU = (NMT + 3) / 4;  // chunks of 8 k of one slot a thread stages
+    // chunk it = tid + 256 u: slot it / 4, lane group it mod 4; slots past n are zero
+    const int sg = tid & 3;
+    const float* ap[NU];
+    bool aok[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int slot = (tid >> 2) + 64 * u;
+      aok[u] = slot < n;
+      ap[u] = A + (m0 + prow[aok[u] ? slot : 0]) * K;
+    }
+    const int bn[2] = {n0 + wn + c < N ? n0 + wn + c : N - 1, n0 + wn + 16 + c < N ? n0 + wn + 16 + c : N - 1};
+    float4 ra[NU][2];
+    float rb[2][8];
+    // zeros past K in A; B repeats its last row there
+    auto gload = [&](int k0) {
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+          const int kk = k0 + 8 * sg + 4 * v;
+          ra[u][v] = make_float4(0.f, 0.f, 0.f, 0.f);
+          if (aok[u] && kk < K) ra[u][v] = *reinterpret_cast<const float4*>(ap[u] + kk);
+        }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int kk = k0 + 8 * g + j;
+        const float* const br = Bm + static_cast<int64_t>(kk < K ? kk : K - 1) * N;
+        rb[0][j] = br[bn[0]];
+        rb[1][j] = br[bn[1]];
+      }
+    };
+    auto sstore = [&]() {
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        const int slot = (tid >> 2) + 64 * u;
+        const float x[8] = {ra[u][0].x, ra[u][0].y, ra[u][0].z, ra[u][0].w,
+                            ra[u][1].x, ra[u][1].y, ra[u][1].z, ra[u][1].w};
+        const Split8 sp = split8(x);
+        v4u* const d = As + (slot >> 4) * (3 * 64) + 16 * sg + ((slot & 15) ^ (2 * sg));
+        d[0] = sp.h;
+        d[64] = sp.m;
+        d[128] = sp.l;
+      }
+    };
     v4f acc[NMT][2];
 #pragma unroll
     for (int mt = 0; mt < NMT; ++mt) acc[mt][0] = acc[mt][1] = zero4();
-    const int nk = (K + kBK - 1) / kBK;
+    const v4u* const rd = As + 16 * g + (c ^ (2 * g));
     gload(0);
-    sstore(0);
-    __syncthreads();
-    for (int kt = 0; kt < nk; ++kt) {
-      const int buf = kt & 1;
-      if (kt + 1 < nk) gload((kt + 1) * kBK);
-#pragma unroll
-      for (int ks = 0; ks < kBK; ks += 4) {
-        const float b0 = Bs[buf][ks + g][wn + c];
-        const float b1 = Bs[buf][ks + g][wn + 16 + c];
-#pragma unroll
-        for (int mt = 0; mt < NMT; ++mt) {
-          const float af = As[buf][ks + g][(16 * mt + c) ^ (16 * ((ks >> 2) & 3))];
-          acc[mt][0] = mfma16x4(af, b0, acc[mt][0]);
-          acc[mt][1] = mfma16x4(af, b1, acc[mt][1]);
-        }
-      }
-      if (kt + 1 < nk) sstore(buf ^ 1);
+    for (int k0 = 0; k0 < K; k0 += kRK) {
+      if (k0 > 0) __syncthreads();  // the last slice's readers are done
+      sstore();
+      const Split8 b0 = split8(rb[0]), b1 = split8(rb[1]);
       __syncthreads();
+      if (k0 + kRK < K) gload(k0 + kRK);
+      mm_step<NMT>(rd, b0, b1, acc);
     }
     // lane (g, c) holds C[prow[16 mt + 4 g + r]][n0 + wn + 16 nt + c]
+    bool bad = false;
 #pragma unroll
     for (int mt = 0; mt < NMT; ++mt)
 #pragma unroll
@@ -499,9 +492,23 @@ gemm_rows_f32_kernel(const float* __restrict__ A, const float* __restrict__ Bm, 
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
           const int col = n0 + wn + 16 * nt + c;
+          bad |= !finite_f32(acc[mt][nt][r]);
           if (slot < n && col < N) C[row * N + col] = acc[mt][nt][r];
         }
       }
+    if (__any(bad)) {  // formed again in float32; a lane reads back only what it stored
+#pragma unroll 1
+      for (int e = 0; e < 8 * NMT; ++e) {
+        const int slot = 16 * (e >> 3) + 4 * g + (e & 3), col = n0 + wn + 16 * ((e >> 2) & 1) + c;
+        if (slot >= n || col >= N) continue;
+        const int64_t row = m0 + prow[slot];
+        if (finite_f32(C[row * N + col])) continue;
+        float v = 0.f;
+#pragma unroll 1
+        for (int k = 0; k < K; ++k) v = fmaf(A[row * K + k], Bm[static_cast<int64_t>(k) * N + col], v);
+        C[row * N + col] = v;
+      }
+    }
   };
   using std::integral_constant;
   switch ((n + 15) >> 4) {
@@ -876,9 +883,9 @@ __global__ void __launch_bounds__(256) leaf_pair_level_kernel(const float* __res
   }
 }
 
-// Whether the basis serves: at least one pair (and no more than a grid's second dimension), inputs that fit its one K step, and no more basis
-// rows than walker rows, neither at the leaves (2 nq: the basis is held in half a leaf buffer) nor
-// at the pairs (nq^2). At that line (16 walkers, nq = 4, fine-tune widths) the whole wavefunction
+// Whether the basis serves: at least one pair (and no more than a grid's second dimension), inputs
+// that fit its one K step, and no more basis rows than walker rows, neither at the leaves (2 nq: the
+// basis is held in half a leaf buffer) nor at the pairs (nq^2). At that line (16 walkers, nq = 4, fine-tune widths) the whole wavefunction
 // takes 948 -> 732 us at 64 sites and 660 -> 456 us at 8; 500 x 64 sites 4618 -> 1978 us, 1024 x 64
 // 8799 -> 3386 us.
 bool basis_serves(int64_t B, int n, int nq) {

@@ -98,18 +98,18 @@ template <int MB>
 __device__ __forceinline__ void mm_step(const v4u* W, const Split8& b0, const Split8& b1, v4f (&acc)[MB][2]) {
   const bf16x8 b[2][3] = {{as_bf16x8(b0.h), as_bf16x8(b0.m), as_bf16x8(b0.l)},
                           {as_bf16x8(b1.h), as_bf16x8(b1.m), as_bf16x8(b1.l)}};
-  constexpr int G = MB % 2 == 0 ? 2 : 1;
+  constexpr int G = MB >= 2 ? 2 : 1;
 #pragma unroll
   for (int m0 = 0; m0 < MB; m0 += G) {
     bf16x8 a[G][3];
 #pragma unroll
-    for (int i = 0; i < G; ++i)
+    for (int i = 0; i < G && m0 + i < MB; ++i)
 #pragma unroll
       for (int part = 0; part < 3; ++part) a[i][part] = as_bf16x8(W[((m0 + i) * 3 + part) * 64]);
 #pragma unroll
     for (int t = 0; t < kSplitTerms; ++t)
 #pragma unroll
-      for (int i = 0; i < G; ++i)
+      for (int i = 0; i < G && m0 + i < MB; ++i)
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb)
           acc[m0 + i][cb] = mfma16_bf16(a[i][kSplitA[t]], b[cb][kSplitB[t]], acc[m0 + i][cb]);

@@ -239,6 +239,40 @@ def test_out_proj_masked_row_compaction():
     assert np.all(delta.cpu().numpy()[~mask] == 0.0) and np.all(dt[0].cpu().numpy()[~mask] == 0.0)
 
 
+@pytest.mark.parametrize("hh,D,d_e", [(16, 16, 8196), (5, 4, 8320), (3, 12, 8196)])
+def test_out_proj_row_kernel(hh, D, d_e):
+    """Enough workgroups for the row-compacting kernel (256 rows x 128 columns each, at least one
+    per CU): no, every, one, an odd count of and the last few physical rows in a workgroup,
+    contraction lengths with and without a remainder of 32 (256, 20, 36), a partial column tile;
+    a row with an infinity and one above the largest bfloat16 (whose sums float32 forms)."""
+    from hamiltonzero_amd import kernels
+
+    _say(f"out proj row kernel {hh}x{D} -> {d_e}")
+    rng = np.random.default_rng(hh + d_e)
+    M, K = 1029, hh * D
+    y = rng.standard_normal((M, 1, hh, D), dtype=np.float32)
+    w = (rng.standard_normal((K, d_e)) / np.sqrt(K)).astype(np.float32)
+    mask = np.zeros((M, 1), dtype=bool)
+    mask[256:512] = True
+    mask[512 + 77] = True
+    mask[768 + rng.permutation(256)[:141]] = True
+    mask[1024:1028] = True
+    y[300] = 0.0
+    y[300, 0, 1, 3] = 3.4e38
+    y[301, 0, 2, 1] = np.inf
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()  # noqa: E731
+    delta, _ = kernels.gated_out_proj(dev(y), dev(w), mask=dev(mask))
+    torch.cuda.synchronize()
+    got = delta.cpu().numpy().reshape(M, d_e)
+    want = y.reshape(M, K).astype(np.float64) @ w.astype(np.float64)
+    assert np.array_equal(got[301], want[301])
+    assert rel(got[300], want[300]) <= TOL
+    rows = mask[:, 0].copy()
+    rows[[300, 301]] = False
+    assert rel(got[rows], want[rows]) <= TOL
+    assert np.all(got[~mask[:, 0]] == 0.0)
+
+
 def test_gated_then_out_proj_at_the_trunk_shape():
     """The trunk's attention tail: gated fwd+JVP at [48, 64, 32, 16] with bias, then W_O
     [256, 512] on y and ydot, against the oracle's chain."""
