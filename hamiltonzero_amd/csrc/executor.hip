@@ -362,7 +362,7 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ Bm, float
 // all threads, into 48 KB of LDS that every wave reads; a wave's columns of B come from memory to its
 // registers and are split there, a slice ahead of their products. Two workgroups of 50 KB and 244
 // registers a CU, so one stages under the other's products. Bound by memory (its output alone is
-// 134 MB) and the splits: 65536 rows, 36 of 64 physical, 256 x 512, y and its tangent 210 -> 151 us
+// 134 MB) and the splits: 65536 rows, 36 of 64 physical, 256 x 512, y and its tangent 214 -> 155 us
 // (the float32 matrix instruction was 53% busy).
 constexpr int kRM = 256;  // 16 row blocks: the dispatch below instantiates 1..16
 constexpr int kRK = 32;   // K per slice: one matrix step
@@ -1018,6 +1018,8 @@ hipError_t launch_out_proj(const float* y, const float* w_o, const uint8_t* mask
   // rows, e.g. one large-N system's 4096 query rows: 64 workgroups for 256 CUs) the 128 x 128
   // tiled GEMM with the row mask in its epilogue runs twice the workgroups and multiplies the
   // masked rows too (the large-N tail's W_O on 4096 rows: about 93 -> 53 us).
+  // At the line (16384 rows, 512 columns) the row kernel takes 29 us with 36 of 64 rows physical and
+  // 40 with all, the tiled one 39 and 38; at 65536 rows 86 and 106 against 142 and 133.
   int cus = 0;
   if (hipError_t err = device_cu_count(&cus); err != hipSuccess) return err;
   const int64_t ncol = (d_out + kBN - 1) / kBN;
