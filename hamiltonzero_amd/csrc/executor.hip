@@ -737,40 +737,201 @@ __global__ void __launch_bounds__(256) readout_kernel(const float* __restrict__ 
 // The leaf and the first level through a basis of the walkers' inputs
 // --------------------------------------------------------------------------------------
 // Everything from a site's input q [nq] to the first merge is linear in q: the leaf carrier is
-// u = sum_c q_c E[c], E[c] = ((W_q[c] V) o h) U, and a node of the first level is bilinear,
-// out = sum_cd q_c q'_d O[c, d] with O the level's merge and residual apply of E[c] and E'[d].
-// So the leaf's and the first level's products run on nq rows per leaf and nq^2 rows per pair
-// instead of on every walker's rows, and this kernel forms each walker's carrier from them: the
-// leaf carriers' norms, the normalised coefficients, the node's sum, its rescale and its gate
-// (normalize_rows_kernel and level_gate_kernel of the plain path). At 1024 walkers of 64 sites
-// with nq = 4 the products fall from 65536 leaf and 32768 pair rows to 256 and 512.
-// A workgroup owns 16 walkers of one node pair p, its waves a quarter of the columns each.
-// Orientation: basis columns x walkers on
-// v_mfma_f32_16x16x4_f32, the contraction over c (leaf) or, in four steps, over (c, d); the row
-// of 16 columns a lane's register holds is one 16-byte store, 64 bytes per walker. Three passes
-// over the columns: leaf norms, the node's norm, the stores (the sums are formed again: the
-// basis is in L2 and the products are few). 107 us at 1024 x 64 sites, 41 of them for the 201 MB of
-// carriers it writes (139 us with a wave per 16 walkers and every column: too few waves).
+// u = sum_c q_c E[c], E[c] = ((W_q[c] V) o h) U, and a node of the first level is bilinear in the two
+// leaves' inputs. So the leaf's and the first level's products run on nq rows per leaf and nq^2
+// rows per pair instead of on every walker's rows. At 1024 walkers of 64 sites with nq = 4 the
+// products fall from 65536 leaf and 32768 pair rows to 256 and 512.
+// A sum over E itself would lose what the inputs cancel (a carrier kappa times smaller than its
+// terms), and a node the product of what its two leaves cancel. So E is formed in 64 bits and each
+// leaf's rows are made orthonormal there (orthonormal_basis_kernel): E[c] = sum_a R[a, c] Q[a] with
+// mean(Q[a] Q[b]) = (a == b). A walker's coefficients y = R q are 64-bit sums, its carrier's rms is
+// |y|, and the node is out = sum_ab (y_a / |y|) (y'_b / |y'|) O[a, b] with O the level's merge and
+// residual apply of Q[a] and Q'[b]: terms of the node's own size, whatever q cancels. The node's
+// error against 64 bits stays below 1e-6 for inputs that cancel by up to 1e5, where the products on
+// every walker's rows lose 2.6e-3.
 constexpr int kMaxBasis = 4;  // inputs per site the pair basis serves (one K step of the products)
 
+typedef double v4d __attribute__((ext_vector_type(4)));
+
 __global__ void __launch_bounds__(256) leaf_basis_kernel(const float* __restrict__ Wq, const float* __restrict__ V,
-                                                         const float* __restrict__ h, float* __restrict__ out, int n,
+                                                         const float* __restrict__ h, double* __restrict__ out, int n,
                                                          int d_z, int R) {
   // out[(c n + s) R + r] = (sum_z W_q[c, z] V[z, r]) h[s, r]
   const int r = blockIdx.x * 256 + threadIdx.x;
   if (r >= R) return;
   const int c = blockIdx.y;
-  float a = 0.f;
-  for (int z = 0; z < d_z; ++z) a = fmaf(Wq[c * d_z + z], V[static_cast<int64_t>(z) * R + r], a);
+  double a = 0.0;
+#pragma unroll 8
+  for (int z = 0; z < d_z; ++z)
+    a = fma(static_cast<double>(Wq[static_cast<int64_t>(c) * d_z + z]),
+            static_cast<double>(V[static_cast<int64_t>(z) * R + r]), a);
   for (int s = blockIdx.z; s < n; s += gridDim.z)
     out[(static_cast<int64_t>(c) * n + s) * R + r] = a * h[static_cast<int64_t>(s) * R + r];
 }
 
-__global__ void __launch_bounds__(256) leaf_pair_level_kernel(const float* __restrict__ E, const float* __restrict__ O,
-                                                               const float* __restrict__ q,
-                                                               const uint8_t* __restrict__ opcodes,
-                                                               float* __restrict__ u_out, float* __restrict__ s_out,
-                                                               int64_t B, int n, int nq, int d, float eps) {
+// C[M, N] = A[M, K] B[K, N] in 64 bits, B held in 32 (the leaf basis times the leaf's U). A workgroup
+// owns 16 rows x 32 columns, its four waves every fourth K block of 16 each, summed through LDS in
+// order. v_mfma_f64_16x16x4_f64, lane l = 16 g + c: A[row c][k g], B[k g][col c], C/D element r at
+// [row g + 4 r][col c]; a lane's four k of a block are 4 g .. 4 g + 3 in both operands, its two columns
+// neighbours. N is a multiple of 32. 39 us for 256 x 1536 x 1536 (15 at the 64-bit matrix rate): few
+// workgroups, each waiting for its operands.
+__global__ void __launch_bounds__(256) basis_gemm_f64_kernel(const double* __restrict__ A, const float* __restrict__ Bm,
+                                                             double* __restrict__ C, int64_t M, int N, int K) {
+  __shared__ double part[4][8][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, c = lane & 15;
+  const int64_t m0 = static_cast<int64_t>(blockIdx.y) * 16;
+  const int n0 = blockIdx.x * 32;
+  const double* const ar = A + (m0 + c < M ? m0 + c : M - 1) * K;  // rows past M repeat the last, not stored
+  const float* const bc = Bm + n0 + 2 * c;
+  v4d acc[2] = {v4d{0.0, 0.0, 0.0, 0.0}, v4d{0.0, 0.0, 0.0, 0.0}};
+  auto step = [&](double a, float b0, float b1) {
+    acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, static_cast<double>(b0), acc[0], 0, 0, 0);
+    acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, static_cast<double>(b1), acc[1], 0, 0, 0);
+  };
+  const int whole = K / 16;
+  // a block's operands, loaded under the products of the one before
+  double a[4], an[4];
+  float2 b[4], bn[4];
+  auto load = [&](int t, double (&a)[4], float2 (&b)[4]) {
+    const int k0 = 16 * t + 4 * g;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      a[j] = ar[k0 + j];
+      b[j] = *reinterpret_cast<const float2*>(bc + static_cast<int64_t>(k0 + j) * N);
+    }
+  };
+  if (wave < whole) load(wave, a, b);
+  for (int t = wave; t < whole; t += 4) {
+    load(t + 4 < whole ? t + 4 : t, an, bn);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) step(a[j], b[j].x, b[j].y);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      a[j] = an[j];
+      b[j] = bn[j];
+    }
+  }
+  if (whole * 16 < K && wave == (whole & 3)) {  // the last K block, zeros past K
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int k = 16 * whole + 4 * g + j;
+      const float* const bk = bc + static_cast<int64_t>(k < K ? k : 0) * N;
+      step(k < K ? ar[k] : 0.0, k < K ? bk[0] : 0.f, k < K ? bk[1] : 0.f);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    part[wave][2 * r][lane] = acc[0][r];
+    part[wave][2 * r + 1][lane] = acc[1][r];
+  }
+  __syncthreads();
+  // wave w stores element r = w of both blocks
+  const int64_t row = m0 + g + 4 * wave;
+  if (row < M) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int e = 2 * wave + j;
+      C[row * N + n0 + 2 * c + j] = (part[0][e][lane] + part[1][e][lane]) + (part[2][e][lane] + part[3][e][lane]);
+    }
+  }
+}
+
+// One leaf's nq rows E (64 bits, [nq][n][d]) made orthonormal: Q [nq][n][d] in 32 bits with
+// mean(Q_a Q_b) = (a == b), R [n][nq][nq] in 64 bits with E_c = sum_a R[a, c] Q_a (Gram-Schmidt, each
+// row projected twice). A row whose rest is below 2^-40 of itself depends on the rows before it: its
+// Q and its row of R are zeros, and what is left out is 2^-40 of E_c. One workgroup a leaf, a row
+// eight values a thread; d <= 2048.
+__global__ void __launch_bounds__(256) orthonormal_basis_kernel(const double* __restrict__ E, float* __restrict__ Q,
+                                                                double* __restrict__ R, int n, int nq, int d) {
+  constexpr int kPer = 8;
+  __shared__ double red[2][4][kMaxBasis];
+  const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const double inv_d = 1.0 / static_cast<double>(d);
+  int turn = 0;
+  // mean over the row of NV products, in every thread
+  auto means = [&](double (&v)[kMaxBasis], int count) {
+#pragma unroll
+    for (int i = 0; i < kMaxBasis; ++i)
+      if (i < count)
+        for (int off = 32; off > 0; off >>= 1) v[i] += __shfl_xor(v[i], off);
+    if (lane == 0)
+#pragma unroll
+      for (int i = 0; i < kMaxBasis; ++i) red[turn][wave][i] = v[i];
+    __syncthreads();  // (two buffers: the last means' readers are behind this barrier)
+#pragma unroll
+    for (int i = 0; i < kMaxBasis; ++i)
+      v[i] = ((red[turn][0][i] + red[turn][1][i]) + (red[turn][2][i] + red[turn][3][i])) * inv_d;
+    turn ^= 1;
+  };
+  double basis[kMaxBasis][kPer];
+  double* const Rs = R + static_cast<int64_t>(s) * nq * nq;
+#pragma unroll
+  for (int a = 0; a < kMaxBasis; ++a) {
+    if (a >= nq) break;
+    const int64_t at = (static_cast<int64_t>(a) * n + s) * d;
+    double x[kPer], r[kMaxBasis] = {0.0, 0.0, 0.0, 0.0}, v[kMaxBasis] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int col = tid + 256 * i;
+      x[i] = col < d ? E[at + col] : 0.0;
+      v[0] = fma(x[i], x[i], v[0]);
+    }
+    means(v, 1);
+    const double before = v[0];
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+      if (a == 0) break;
+#pragma unroll
+      for (int b = 0; b < a; ++b) {
+        v[b] = 0.0;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) v[b] = fma(basis[b][i], x[i], v[b]);
+      }
+      means(v, a);
+#pragma unroll
+      for (int b = 0; b < a; ++b) {
+        r[b] += v[b];
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) x[i] = fma(-v[b], basis[b][i], x[i]);
+      }
+    }
+    v[0] = 0.0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) v[0] = fma(x[i], x[i], v[0]);
+    means(v, 1);
+    // (also a row of zeros; not one with a value that is not finite, which stays so)
+    const bool none = before < __builtin_huge_val() && v[0] <= before * 0x1p-80;
+    const double norm = none ? 0.0 : sqrt(v[0]), inv = none ? 0.0 : 1.0 / norm;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      basis[a][i] = x[i] * inv;
+      const int col = tid + 256 * i;
+      if (col < d) Q[at + col] = static_cast<float>(basis[a][i]);
+    }
+    if (tid < nq) {  // column a of R, by row; zeros below the diagonal
+      double v_r = tid == a ? norm : 0.0;
+#pragma unroll
+      for (int b = 0; b < a; ++b)
+        if (tid == b) v_r = r[b];
+      Rs[tid * nq + a] = v_r;
+    }
+  }
+}
+
+// The walkers' carriers after the first level, from the orthonormal basis Q, its pairs' nodes O and R:
+// the leaf carriers' norms and coefficients, the node's sum, its rescale and its gate
+// (normalize_rows_kernel and level_gate_kernel of the plain path). A workgroup owns 16 walkers of one
+// node pair p, its waves a quarter of the columns each. Orientation: basis columns x walkers on
+// v_mfma_f32_16x16x4_f32, the contraction over a (leaf) or, in four steps, over (a, b); the row of 16
+// columns a lane's register holds is one 16-byte store, 64 bytes per walker. Two passes over the
+// columns: the node's norm, the stores (the sums are formed again: the basis is in L2 and the
+// products are few). 100 us at 1024 x 64 sites, 41 of them for the 201 MB of carriers it writes.
+__global__ void __launch_bounds__(256) leaf_pair_level_kernel(const float* __restrict__ Q, const float* __restrict__ O,
+                                                              const double* __restrict__ R, const float* __restrict__ q,
+                                                              const uint8_t* __restrict__ opcodes,
+                                                              float* __restrict__ u_out, float* __restrict__ s_out,
+                                                              int64_t B, int n, int nq, int d, float eps) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
   const int p = blockIdx.y, w = n / 2;
@@ -779,58 +940,39 @@ __global__ void __launch_bounds__(256) leaf_pair_level_kernel(const float* __res
   // this wave's columns, in steps of 32 (d is a multiple of 32)
   const int steps = d / 32;
   const int t0 = 32 * (steps * wave / 4), t1 = 32 * (steps * (wave + 1) / 4);
-  __shared__ float part[3][4][16];  // per wave and walker: sums of squares (left leaf, right leaf, node)
-  float ql[kMaxBasis], qr[kMaxBasis];
+  __shared__ float part[4][16];  // per wave and walker: the node's sum of squares
+  // y = R q of one leaf over its rms, which is sqrt(mean(u^2) + 1e-30) with mean(u^2) = |y|^2
+  auto coefficients = [&](int leaf, float (&y)[kMaxBasis]) {
+    const float* const qb = q + ((ok ? b : 0) * n + leaf) * nq;
+    const double* const Rl = R + static_cast<int64_t>(leaf) * nq * nq;
+    double yd[kMaxBasis], ss = 0.0;
 #pragma unroll
-  for (int s = 0; s < kMaxBasis; ++s) {
-    const float* qb = q + ((ok ? b : 0) * n + 2 * p) * nq;
-    ql[s] = s < nq ? qb[s] : 0.f;
-    qr[s] = s < nq ? qb[nq + s] : 0.f;
-  }
+    for (int a = 0; a < kMaxBasis; ++a) {
+      yd[a] = 0.0;
+#pragma unroll
+      for (int i = 0; i < kMaxBasis; ++i)
+        if (a < nq && i < nq) yd[a] = fma(Rl[a * nq + i], static_cast<double>(qb[i]), yd[a]);
+      ss = fma(yd[a], yd[a], ss);
+    }
+    const double rms = sqrt(ss + 1e-30);
+#pragma unroll
+    for (int a = 0; a < kMaxBasis; ++a) y[a] = static_cast<float>(yd[a] / rms);
+    return static_cast<float>(rms);
+  };
+  float yl[kMaxBasis], yr[kMaxBasis];
+  const float rl = coefficients(2 * p, yl), rr = coefficients(2 * p + 1, yr);
+  auto lane_of = [&](const float (&x)[kMaxBasis]) { return g == 0 ? x[0] : (g == 1 ? x[1] : (g == 2 ? x[2] : x[3])); };
+  const float bl = lane_of(yl), br = lane_of(yr);
+  float co[kMaxBasis];
+#pragma unroll
+  for (int s = 0; s < kMaxBasis; ++s) co[s] = yl[s] * br;
   // this lane group's basis row; past nq (coefficient 0) any row
   const int gr = g < nq ? g : 0;
-  const float* El = E + (static_cast<int64_t>(gr) * n + 2 * p) * d + c;
-  const float* Er = El + d;
+  const float* Ql = Q + (static_cast<int64_t>(gr) * n + 2 * p) * d + c;
+  const float* Qr = Ql + d;
   const float* Os[kMaxBasis];
 #pragma unroll
   for (int s = 0; s < kMaxBasis; ++s) Os[s] = O + (static_cast<int64_t>((s < nq ? s : 0) * nq + gr) * w + p) * d + c;
-  auto lane_of = [&](const float (&x)[kMaxBasis]) { return g == 0 ? x[0] : (g == 1 ? x[1] : (g == 2 ? x[2] : x[3])); };
-
-  // leaf carriers' norms: rms = sqrt(mean(u^2) + 1e-30)
-  float bl = lane_of(ql), br = lane_of(qr);
-  float ssl = 0.f, ssr = 0.f;
-  for (int t = t0; t < t1; t += 32) {
-    float al[2], ar[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      al[j] = El[t + 16 * j];
-      ar[j] = Er[t + 16 * j];
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const v4f ul = mfma16x4(al[j], bl, zero4()), ur = mfma16x4(ar[j], br, zero4());
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        ssl = fmaf(ul[r], ul[r], ssl);
-        ssr = fmaf(ur[r], ur[r], ssr);
-      }
-    }
-  }
-  ssl = group_sum(ssl);
-  ssr = group_sum(ssr);
-  if (g == 0) {
-    part[0][wave][c] = ssl;
-    part[1][wave][c] = ssr;
-  }
-  __syncthreads();
-  auto whole = [&](int i) { return (part[i][0][c] + part[i][1][c]) + (part[i][2][c] + part[i][3][c]); };
-  const float fd = static_cast<float>(d);
-  const float rl = sqrtf(whole(0) / fd + 1e-30f), rr = sqrtf(whole(1) / fd + 1e-30f);
-  bl /= rl;
-  br /= rr;
-  float co[kMaxBasis];
-#pragma unroll
-  for (int s = 0; s < kMaxBasis; ++s) co[s] = ql[s] / rl * br;
   // the node's sum in columns t .. t + 31
   auto node = [&](int t, v4f (&o)[2]) {
     float a[2][kMaxBasis];
@@ -855,9 +997,10 @@ __global__ void __launch_bounds__(256) leaf_pair_level_kernel(const float* __res
       for (int r = 0; r < 4; ++r) ss = fmaf(o[j][r], o[j][r], ss);
   }
   ss = group_sum(ss);
-  if (g == 0) part[2][wave][c] = ss;
+  if (g == 0) part[wave][c] = ss;
   __syncthreads();
-  const float scale = sqrtf(whole(2) / fd + eps);
+  const float whole = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+  const float scale = sqrtf(whole / static_cast<float>(d) + eps);
   const float inv = 1.0f / scale;
   const int op = opcodes[p];
   const float both = op == 0 ? 1.f : 0.f, left = op == 1 ? 1.f : 0.f, right = op == 2 ? 1.f : 0.f;
@@ -870,7 +1013,7 @@ __global__ void __launch_bounds__(256) leaf_pair_level_kernel(const float* __res
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[j][r] *= inv;
       if (op != 0) {
-        const v4f ul = mfma16x4(El[t + 16 * j], bl, zero4()), ur = mfma16x4(Er[t + 16 * j], br, zero4());
+        const v4f ul = mfma16x4(Ql[t + 16 * j], bl, zero4()), ur = mfma16x4(Qr[t + 16 * j], br, zero4());
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[j][r] = both * o[j][r] + left * ul[r] + right * ur[r];
       }
@@ -885,11 +1028,13 @@ __global__ void __launch_bounds__(256) leaf_pair_level_kernel(const float* __res
 
 // Whether the basis serves: at least one pair (and no more than a grid's second dimension), inputs
 // that fit its one K step, and no more basis rows than walker rows, neither at the leaves (2 nq: the
-// basis is held in half a leaf buffer) nor at the pairs (nq^2). At that line (16 walkers, nq = 4, fine-tune widths) the whole wavefunction
-// takes 948 -> 732 us at 64 sites and 660 -> 456 us at 8; 500 x 64 sites 4618 -> 1978 us, 1024 x 64
-// 8799 -> 3386 us.
-bool basis_serves(int64_t B, int n, int nq) {
-  return n > 1 && n / 2 <= 65535 && nq <= kMaxBasis && B >= static_cast<int64_t>(nq) * nq && B >= 2 * nq;
+// basis in 64 bits and its factors take half a leaf buffer each as floats) nor at the pairs (nq^2);
+// R in 64 bits fits where z is not needed. At that line (nq = 4, fine-tune widths) the whole
+// wavefunction takes 319 us for 16 walkers of 8 sites with it and 436 for 15 without, 532 and 657
+// at 64 sites.
+bool basis_serves(int64_t B, int n, int nq, int d_z) {
+  const int64_t nq2 = static_cast<int64_t>(nq) * nq;
+  return n > 1 && n / 2 <= 65535 && nq <= kMaxBasis && B >= nq2 && B >= 2 * nq && B * d_z >= 2 * nq2;
 }
 
 hipError_t launch_merge(const float* T, const float* ua, const float* ub, float* out, int64_t M, int G,
@@ -940,17 +1085,24 @@ hipError_t launch_compiled_wavefunction(const WaveFnParams& p, hipStream_t strea
   const int G = p.d_m / kQR;
   hipError_t err;
   int cur = 0, level = 0, width = p.n / 2;
-  if (basis_serves(p.B, p.n, p.d_q)) {
-    // E in the second carrier buffer, the first level's node basis in raw, carriers into the first
+  if (basis_serves(p.B, p.n, p.d_q, p.d_z)) {
+    // E in 64 bits in the first carrier buffer (its left factor in work), Q in the second, R in z, the
+    // first level's node basis in raw, carriers into the first
     const int64_t er = static_cast<int64_t>(p.d_q) * p.n, pr = static_cast<int64_t>(p.d_q) * p.d_q * width;
+    double *const factor = reinterpret_cast<double*>(work), *const E = reinterpret_cast<double*>(u_buf[0]);
+    double* const R = reinterpret_cast<double*>(z);
     hipLaunchKernelGGL(leaf_basis_kernel,
                        dim3(static_cast<unsigned>((p.r_leaf + 255) / 256), static_cast<unsigned>(p.d_q),
                             static_cast<unsigned>(p.n < 16 ? p.n : 16)),
-                       dim3(256), 0, stream, p.q_weight, p.leaf_V, p.leaf_h, work, p.n, p.d_z, p.r_leaf);
+                       dim3(256), 0, stream, p.q_weight, p.leaf_V, p.leaf_h, factor, p.n, p.d_z, p.r_leaf);
     if ((err = hipGetLastError()) != hipSuccess) return err;
-    if ((err = launch_gemm<kEpiPlain>(work, p.leaf_U, u_buf[1], nullptr, er, p.d_m, p.r_leaf, 1, 0, stream, u_buf[0],
-                                      u_cap[0])) != hipSuccess)
-      return err;
+    hipLaunchKernelGGL(basis_gemm_f64_kernel,
+                       dim3(static_cast<unsigned>(p.d_m / 32), static_cast<unsigned>((er + 15) / 16)), dim3(256), 0,
+                       stream, factor, p.leaf_U, E, er, p.d_m, p.r_leaf);
+    if ((err = hipGetLastError()) != hipSuccess) return err;
+    hipLaunchKernelGGL(orthonormal_basis_kernel, dim3(static_cast<unsigned>(p.n)), dim3(256), 0, stream, E, u_buf[1], R,
+                       p.n, p.d_q, p.d_m);
+    if ((err = hipGetLastError()) != hipSuccess) return err;
     if ((err = launch_merge(p.merge_T, u_buf[1], u_buf[1], raw, pr, G, MergeRows{p.d_m, width, p.d_q, p.n}, stream)) !=
         hipSuccess)
       return err;
@@ -959,7 +1111,7 @@ hipError_t launch_compiled_wavefunction(const WaveFnParams& p, hipStream_t strea
       return err;
     hipLaunchKernelGGL(leaf_pair_level_kernel,
                        dim3(static_cast<unsigned>((p.B + 15) / 16), static_cast<unsigned>(width)), dim3(256), 0, stream,
-                       u_buf[1], raw, p.q, p.opcodes, u_buf[0], s_buf[0], p.B, p.n, p.d_q, p.d_m, p.merge_eps);
+                       u_buf[1], raw, R, p.q, p.opcodes, u_buf[0], s_buf[0], p.B, p.n, p.d_q, p.d_m, p.merge_eps);
     if ((err = hipGetLastError()) != hipSuccess) return err;
     level = 1;
     width /= 2;

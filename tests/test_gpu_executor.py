@@ -270,6 +270,36 @@ def test_compiled_wavefunction_pair_basis(B, n, d_q, G, real):
     assert np.all(dphi <= TOL * np.pi + 1e-6 * kappa), (dphi.max(), kappa[np.argmax(dphi)])
 
 
+@pytest.mark.parametrize("rows", ["1e-1", "1e-2", "1e-3", "equal", "zero"])
+def test_pair_basis_of_inputs_that_cancel(rows):
+    """Leaves whose inputs cancel: the rows of q_to_odd are a common vector and a part of size
+    ``rows`` of their own, and a site's inputs sum to zero, so its carrier is about 1 / rows times
+    smaller than the carriers of its single inputs. The same bound as for inputs that do not
+    cancel: the carrier is a function of q to be evaluated, not of rounded sums. Rows that are
+    equal, or zero, leave a basis of fewer rows."""
+    from hamiltonzero_amd import executor
+
+    _say(f"wavefunction basis, cancelling inputs, rows {rows}")
+    B, n, d_q, G = 33, 4, 4, 4
+    p = _wavefn_case(5, B, n, d_q, 32, 256, G, 128, 12, "all")
+    rng = np.random.default_rng(9)
+    if rows in ("equal", "zero"):
+        p["q_weight"][2:] = p["q_weight"][0] if rows == "equal" else 0.0
+    else:
+        own = rng.standard_normal((d_q, 32)) * float(rows)
+        p["q_weight"] = ((rng.standard_normal(32) + own) / 2).astype(np.float32)
+        p["q"][..., 1], p["q"][..., 3] = -p["q"][..., 0], -p["q"][..., 2]
+    kernel, tree, q = _namespaces(p)
+    la, ph = executor.execute_wavefunction(kernel, tree, q)
+    torch.cuda.synchronize()
+    want_la, want_ph = X.execute_wavefunction(**p)
+    kappa = _readout_condition(p)
+    dla = np.abs(la.cpu().numpy().astype(np.float64) - want_la)
+    assert np.all(dla <= TOL * np.max(np.abs(want_la)) + 1e-6 * kappa), (dla.max(), kappa[np.argmax(dla)])
+    dphi = np.abs(np.angle(np.exp(1j * (ph.cpu().numpy().astype(np.float64) - want_ph))))
+    assert np.all(dphi <= TOL * np.pi + 1e-6 * kappa), (dphi.max(), kappa[np.argmax(dphi)])
+
+
 def test_compiled_wavefunction_structure_errors():
     from hamiltonzero_amd import executor
 
