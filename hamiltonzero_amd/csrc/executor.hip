@@ -151,21 +151,36 @@ quadrilinear_merge_kernel(const float* __restrict__ T, const float* __restrict__
   bool bad = false;
 #pragma unroll
   for (int e = 0; e < 16; ++e) bad |= !finite_f32(acc[e]);
-  if (__any(bad)) {  // formed again in float32 (through LDS: an index known at run time)
-    float* const mine = reinterpret_cast<float*>(&Ts[0][0][0][0][0]) + wave * 1024 + lane;
+  if (__any(bad)) {  // formed again in float32, unless a NaN of the row's operands made them
+    bool nan = false;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) mine[64 * e] = acc[e];
-#pragma unroll 1
-    for (int e = 0; e < 16; ++e) {
-      if (finite_f32(mine[64 * e]) || row >= M) continue;
-      const float* tj = T + (static_cast<int64_t>(i) * kQR + 8 * (e >> 2) + 4 * hh + (e & 3)) * kQR * kQR;
-      float v = 0.f;
-#pragma unroll 1
-      for (int kl = 0; kl < kQR * kQR; ++kl) v = fmaf(ar[kl >> 5] * br[kl & 31], tj[kl], v);
-      mine[64 * e] = v;
+    for (int q = 0; q < kQR / 4; ++q) {
+      const v4f x = *reinterpret_cast<const v4f*>(ar + 4 * q), y = *reinterpret_cast<const v4f*>(br + 4 * q);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) nan |= x[u] != x[u] || y[u] != y[u];
     }
+    bad = bad && !nan && row < M;
+    if (__any(bad)) {
+      const float* const tj = T + (static_cast<int64_t>(i) * kQR + c) * kQR * kQR + 4 * hh;
+      v16f w = v16f{};
+#pragma unroll 1
+      for (int k = 0; k < kQR; ++k) {
+        const float ak = ar[k];
+        v4f t[4], y[4];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = mine[64 * e];
+        for (int q = 0; q < 4; ++q) {
+          t[q] = *reinterpret_cast<const v4f*>(tj + k * kQR + 8 * q);
+          y[q] = *reinterpret_cast<const v4f*>(br + 4 * hh + 8 * q);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) w = mfma32_f32(t[q][u], ak * y[q][u], w);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (bad && !finite_f32(acc[e])) acc[e] = w[e];
+    }
   }
   if (row < M) {
 #pragma unroll
@@ -200,6 +215,10 @@ enum GemmEpi { kEpiPlain = 0, kEpiCond = 1, kEpiResidual = 2, kEpiRowMask = 3 };
 // the same row), the slice's columns of B through LDS, double-buffered, as their three bfloat16
 // parts: a column is 2 chunks of 8 k (16 bytes, one operand read), chunk h of column n at
 // h ^ ((n / 4) mod 2), which spreads any 8 consecutive lanes of a read or a store over all banks.
+// Sums that are not finite are formed again on the float32 instruction, a wave's 32 x 32 block at a
+// time, unless a NaN in the row of A made them: a diverged walker's row costs nothing, one with an
+// infinity 0.4 ms where the wave comes last (16384 rows, K = 1536; 1.7 ms with a lane's own loop
+// per sum).
 // A thread stages 8 k of one column. Loads run kAhead slices ahead of their products (1024 rows,
 // one workgroup to a CU: 202 us with one slice, 166 with two, 167 with four).
 template <int EPI, bool VEC>
@@ -310,7 +329,55 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ Bm, float
 
   // element i of block nt: row m0 + 8 (i / 4) + 4 hh + i % 4, column n0 + 32 nt + c
   auto row_of = [&](int i) { return m0 + 8 * (i >> 2) + 4 * hh + (i & 3); };
-  float* const mine = reinterpret_cast<float*>(&smem[0][0]) + wave * 1024 + lane;
+  uint32_t top = 0;  // (the largest magnitude: as 64 tests their masks would spill)
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const uint32_t mag = __float_as_uint(acc[nt][i]) & 0x7fffffffu;
+      top = top > mag ? top : mag;
+    }
+  if (__any(top >= 0x7f800000u)) {  // formed again in float32, unless a NaN in the row of A made them
+    const float* const arow = Ap - 8 * hh;
+    bool nan = false;
+#pragma unroll 4
+    for (int k = hh; k < K; k += 2) nan |= arow[k] != arow[k];
+    const uint64_t lanes = __ballot(nan || m0 + c >= M);
+    const unsigned rows = static_cast<unsigned>(lanes | (lanes >> 32)) >> (4 * hh);
+    float* const mine = reinterpret_cast<float*>(&smem[0][0]) + wave * 1024 + lane;  // what stands
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const int col = n0 + 32 * nt + c;
+      bool again = false;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const bool stands = finite_f32(acc[nt][i]) || (rows >> (8 * (i >> 2) + (i & 3)) & 1u) != 0;
+        again |= !stands;
+        mine[64 * i] = stands ? acc[nt][i] : __builtin_inff();
+      }
+      if (!__any(again && col < N)) continue;
+      acc[nt] = v16f{};
+      const float* const bcol = Bm + (col < N ? col : N - 1);
+#pragma unroll 1
+      for (int k0 = 0; k0 < K; k0 += 16) {
+        float x[8], y[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int k = k0 + 8 * hh + u, kc = k < K ? k : K - 1;
+          const float xa = arow[kc], yb = bcol[static_cast<int64_t>(kc) * N];
+          x[u] = k < K ? xa : 0.f;
+          y[u] = k < K ? yb : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc[nt] = mfma32_f32(x[u], y[u], acc[nt]);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float v = mine[64 * i];
+        if (finite_f32(v) || v != v) acc[nt][i] = v;
+      }
+    }
+  }
   unsigned hrow[16];
   if constexpr (EPI == kEpiCond) {
     const unsigned hbase = static_cast<unsigned>((row0 + m0) % h_rows);
@@ -320,24 +387,6 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ Bm, float
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int col = n0 + 32 * nt + c;
-    bool bad = false;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) bad |= !finite_f32(acc[nt][i]);
-    if (__any(bad)) {  // formed again in float32 (through LDS: an index known at run time)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) mine[64 * i] = acc[nt][i];
-#pragma unroll 1
-      for (int i = 0; i < 16; ++i) {
-        const int64_t row = row_of(i);
-        if (finite_f32(mine[64 * i]) || row >= M || col >= N) continue;
-        float v = 0.f;
-#pragma unroll 1
-        for (int k = 0; k < K; ++k) v = fmaf(A[row * lda + k], Bm[static_cast<int64_t>(k) * N + col], v);
-        mine[64 * i] = v;
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[nt][i] = mine[64 * i];
-    }
     if (col >= N) continue;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -496,17 +545,51 @@ gemm_rows_f32_kernel(const float* __restrict__ A, const float* __restrict__ Bm, 
           if (slot < n && col < N) C[row * N + col] = acc[mt][nt][r];
         }
       }
-    if (__any(bad)) {  // formed again in float32; a lane reads back only what it stored
+    // formed again in float32, unless a NaN in the row of A made them (a lane reads back only what it
+    // stored)
+    if (__any(bad)) {
 #pragma unroll 1
-      for (int e = 0; e < 8 * NMT; ++e) {
-        const int slot = 16 * (e >> 3) + 4 * g + (e & 3), col = n0 + wn + 16 * ((e >> 2) & 1) + c;
-        if (slot >= n || col >= N) continue;
-        const int64_t row = m0 + prow[slot];
-        if (finite_f32(C[row * N + col])) continue;
-        float v = 0.f;
+      for (int mt = 0; mt < NMT; ++mt) {
+        unsigned again = 0;  // element 4 nt + r
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int slot = 16 * mt + 4 * g + (e & 3), col = n0 + wn + 16 * (e >> 2) + c;
+          if (slot < n && col < N && !finite_f32(C[(m0 + prow[slot]) * N + col])) again |= 1u << e;
+        }
+        if (!__any(again != 0)) continue;
+        const int slot_a = 16 * mt + c;
+        const float* const arow = A + (m0 + prow[slot_a < n ? slot_a : 0]) * K;
+        bool nan = false;
+#pragma unroll 4
+        for (int k = 4 * g; k < K; k += 16) {
+          const v4f x = *reinterpret_cast<const v4f*>(arow + k);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) nan |= x[u] != x[u];
+        }
+        uint64_t lanes = __ballot(nan);
+        lanes |= lanes >> 32;
+        const unsigned rows = static_cast<unsigned>(lanes | (lanes >> 16)) >> (4 * g);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (rows >> (e & 3) & 1) again &= ~(1u << e);
+        if (!__any(again != 0)) continue;
+        v4f w[2] = {zero4(), zero4()};
 #pragma unroll 1
-        for (int k = 0; k < K; ++k) v = fmaf(A[row * K + k], Bm[static_cast<int64_t>(k) * N + col], v);
-        C[row * N + col] = v;
+        for (int k0 = 0; k0 < K; k0 += 16) {
+          const int k = k0 + 4 * g;
+          v4f x = zero4();
+          if (k < K) x = *reinterpret_cast<const v4f*>(arow + k);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const float* const br = Bm + static_cast<int64_t>(k < K ? k + u : 0) * N;
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt) w[nt] = mfma16x4(x[u], k < K ? br[bn[nt]] : 0.f, w[nt]);
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (again >> e & 1)
+            C[(m0 + prow[16 * mt + 4 * g + (e & 3)]) * N + n0 + wn + 16 * (e >> 2) + c] = w[e >> 2][e & 3];
       }
     }
   };

@@ -29,6 +29,11 @@ __device__ __forceinline__ v16f mfma32_bf16(bf16x8 a, bf16x8 b, v16f c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+// v_mfma_f32_32x32x2_f32, lane l = 32 hh + c: A[row c][k hh], B[k hh][col c]; C/D as above.
+__device__ __forceinline__ v16f mfma32_f32(float a, float b, v16f c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+
 // v_mfma_f32_16x16x32_bf16, lane l = 16 g + c: A[row c][k 8 g + j], B[k 8 g + j][col c], j = 0..7;
 // C/D as v_mfma_f32_16x16x4_f32.
 __device__ __forceinline__ v4f mfma16_bf16(bf16x8 a, bf16x8 b, v4f c) {

@@ -142,6 +142,76 @@ def test_products_of_values_the_split_does_not_hold():
     assert np.all(np.isfinite(got) == mask) and np.all(np.abs(got[mask] - want[mask]) <= TOL * np.abs(want[mask]))
 
 
+@pytest.mark.parametrize("M,d_in,R,d_out", [(1, 5, 3, 2), (33, 37, 50, 131), (129, 48, 260, 64)])
+def test_sums_formed_again(M, d_in, R, d_out):
+    """Rows with an infinity, a NaN or a value above the largest bfloat16, contraction lengths with
+    every remainder, rows and columns past a tile: what float32 arithmetic gives in those rows, and
+    every other row bit for bit what it is without them."""
+    from hamiltonzero_amd import executor
+
+    _say(f"sums formed again M={M} d_in={d_in} R={R} d_out={d_out}")
+    rng = np.random.default_rng(M + d_in)
+    x = rng.random((M, d_in)).astype(np.float32) + 0.5
+    V = rng.random((d_in, R)).astype(np.float32) * 1e-3 + 1e-3
+    U = rng.random((R, d_out)).astype(np.float32) * 1e-3 + 1e-3
+    fac, h = types.SimpleNamespace(V=dev(V), U=dev(U)), dev(np.ones((1, R)))
+    plain = executor._factorized_apply(fac, h, dev(x)).cpu().numpy()
+    put = {0: np.inf, M // 2: 3.4e38, M - 1: -np.inf, M // 3: np.nan}
+    for m, v in put.items():
+        x[m, (3 * m) % d_in] = v
+    got = executor._factorized_apply(fac, h, dev(x)).cpu().numpy()
+    want = X.factorized_apply(V, U, np.ones((1, R)), x)  # every term of a row has one sign
+    for m in range(M):
+        if m not in put:
+            assert np.array_equal(got[m], plain[m]), m
+        elif np.isfinite(want[m]).all():
+            assert np.all(np.abs(got[m] - want[m]) <= TOL * np.abs(want[m])), m
+        else:
+            assert np.array_equal(got[m], want[m].astype(np.float32), equal_nan=True), m
+
+
+@pytest.mark.parametrize("value,most", [(float("nan"), 1.5), (float("inf"), 3.0)])
+def test_a_row_that_is_not_finite_costs_little(value, most):
+    """One walker among 16384 whose row holds a NaN (it has diverged, and carries it through every
+    level): its sums need no second look and the products take their usual time. One with an
+    infinity has its sums formed again by the whole wave (2.4 times the apply's time, two products;
+    a serial loop over the contraction per sum took 3 to 5 times, for a NaN too)."""
+    from hamiltonzero_amd import executor, kernels
+
+    _say(f"cost of a row with {value}")
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    rnd = lambda *s: torch.randn(s, generator=gen, device="cuda")  # noqa: E731
+    M, G, R = 16384, 48, 32
+    T, a, b = rnd(G, R, R, R) / R, rnd(M, G * R), rnd(M, G * R)
+    fac, h = types.SimpleNamespace(V=rnd(G * R, 1024) / 39, U=rnd(1024, G * R) / 32), rnd(1, 1024)
+    y, w_o = rnd(1024, 64, 16, 16), rnd(256, 512) / 16
+    mask = torch.arange(64, device="cuda")[None, :].expand(1024, 64) < 36
+    calls = {
+        "merge": (a, lambda x: executor.quadrilinear_merge(T, x, b)),
+        "apply": (a, lambda x: executor._factorized_apply(fac, h, x)),
+        "out_proj rows": (y, lambda x: kernels.gated_out_proj(x, w_o, mask=mask)[0]),
+        "out_proj tiles": (y, lambda x: kernels.gated_out_proj(x, w_o)[0]),
+    }
+
+    def fastest(fn, x):
+        times = []
+        for _ in range(8):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            fn(x)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    for name, (x, fn) in calls.items():
+        worse = x.clone()
+        worse.view(-1, worse.shape[-1])[77, 5] = value
+        clean, slow = fastest(fn, x), fastest(fn, worse)
+        print(f"{name}: {clean * 1e3:.0f} us, with the row {slow * 1e3:.0f} us", flush=True)
+        assert slow <= most * clean, (name, clean, slow)
+
+
 def test_merge_level_products_compose():
     """One tree level's products as the executor chains them: merge, then the residual apply
     (execute.py:103-104), checked against the oracle's level up to the RMS rescale."""
