@@ -31,7 +31,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from . import kernels
+from . import _native, kernels
 
 Tensor = torch.Tensor
 
@@ -135,9 +135,9 @@ class _MhseaAD(torch.autograd.Function):
 class _GatedAD(torch.autograd.Function):
     """y = sigmoid(out[:, :, :H/2]) * out[:, :, H/2:] of MHSEA(q, k, e, v, mask), the trunk's
     head collapse (trunk.py:134-137). The forward and forward mode run the fused kernel
-    (``hz_mhsea_fwd_jvp_gated``); the calls that want a gradient run :class:`_GatedTrainAD`, so this
-    reverse mode (recomputing (out, lse) for ``hz_mhsea_bwd_gated``) serves only those it leaves
-    here, which the C entry then answers or refuses."""
+    (``hz_mhsea_fwd_jvp_gated``); the calls that want a gradient run :class:`_GatedTrainAD`. A
+    gradient through this one is asked for with the compacted bias layout only (another dtype or
+    an odd H is refused in the forward), which has no reverse mode."""
 
     @staticmethod
     def forward(q, k, e, v, mask, opts):
@@ -149,19 +149,13 @@ class _GatedAD(torch.autograd.Function):
     def setup_context(ctx, inputs, output):
         q, k, e, v, mask, opts = inputs
         ctx.opts = opts
-        ctx.save_for_backward(q, k, e, v, mask)
         ctx.save_for_forward(q, k, e, v, mask)
 
     @staticmethod
     def backward(ctx, dy):
-        q, k, e, v, mask = ctx.saved_tensors
-        scale, key_mask, e_layout = ctx.opts
-        out, lse = kernels.mhsea_fwd(q, k, v, mask, e, scale=scale, key_mask=key_mask, e_layout=e_layout)
-        dq, dk, de, dv = kernels.mhsea_bwd_gated(
-            q, k, v, mask, lse, out, dy.contiguous(), e,
-            want_de=bool(ctx.needs_input_grad[2]), scale=scale, key_mask=key_mask, e_layout=e_layout,
+        raise _native.HzError(
+            _native.HZ_EINVAL, "the compacted bias layout is read by the forward family only: it has no reverse mode"
         )
-        return dq, dk, de, dv, None, None
 
     @staticmethod
     def jvp(ctx, qt, kt, et, vt, _mask_t, _opts_t):

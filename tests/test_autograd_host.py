@@ -6,6 +6,7 @@ import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
 
+from hamiltonzero_amd import _native
 from hamiltonzero_amd import mhsea_tuned as MT
 
 B, N, H, D = 2, 8, 4, 8
@@ -16,6 +17,7 @@ def calls(monkeypatch):
     seen = []
 
     def fwd(q, k, v, mask, e=None, **_):
+        seen.append(("fwd",))
         return torch.ones_like(q), torch.ones(B, N, H)
 
     def bwd(q, k, v, mask, lse, out, dout, e=None, **kw):
@@ -58,6 +60,18 @@ def test_reverse_mode_makes_no_cotangents_of_kept_outputs(calls, monkeypatch, ca
     grads = torch.autograd.grad(y, xs, cot)
     assert torch.equal(given[0][0], cot) and all(d is None for d in given[0][1:])
     assert torch.equal(calls[-1][1], cot) and all(torch.equal(g, torch.ones_like(x)) for g, x in zip(grads, xs))
+
+
+def test_the_compacted_layout_has_no_reverse_mode(calls):
+    """Its forward serves a call that wants a gradient; asking for the gradient is refused at once,
+    without a second attention forward."""
+    (q, k, _, v), mask = operands(True)
+    e = torch.randn(B, H, N, N)
+    y = MT.gated_edge_attention(q, k, e, v, mask, e_layout="compact")
+    calls.clear()
+    with pytest.raises(_native.HzError, match="no reverse mode"):
+        torch.autograd.grad(y, q, torch.ones_like(y))
+    assert not calls
 
 
 @pytest.mark.parametrize("call", list(CALLS))
