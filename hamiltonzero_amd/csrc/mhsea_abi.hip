@@ -652,7 +652,7 @@ int hz_compiled_wavefunction(hipStream_t stream, const float* q, const float* q_
   if (n_sites > 0x7fffffffLL || d_q > 0x7fffffffLL || d_z > 0x7fffffffLL || R_leaf > 0x7fffffffLL ||
       R_merge > 0x7fffffffLL || R_out > 0x7fffffffLL)
     return fail(HZ_EINVAL, "dimensions exceed the 32-bit range");
-  if ((B * n_sites + 127) / 128 > 65535 || (B * n_sites + 127) / 128 > 0x7fffffffLL)
+  if ((B * n_sites + 127) / 128 > 65535)
     return fail(HZ_EINVAL, "B * n_sites = %lld exceeds the grid limit", (long long)(B * n_sites));
   if (!std::isfinite(merge_eps) || merge_eps < 0.0f) return fail(HZ_EINVAL, "merge_eps must be finite and >= 0");
   const int64_t need = hz::compiled_wavefunction_workspace_bytes(B, n_sites, d_z, R_leaf, d_m, R_merge, R_out);
