@@ -262,10 +262,11 @@ def test_attention_never_reads_uncomputed_bias(route):
         assert np.array_equal(a, b, equal_nan=False), name
 
 
-@pytest.mark.parametrize("B,N,H,T", [(3, 7, 16, 1), (2, 64, 32, 1), (4, 33, 64, 0), (70, 18, 32, 1), (2, 130, 16, 0)])
-def test_compact_output_is_zero_where_no_pair_lies(B, N, H, T):
-    """coupling_bias in the compacted layout into memory that held NaN: the pairs of the plain layout
-    (bit for bit) and zeros everywhere else - row pads, tails, walkers with no or one site."""
+@pytest.mark.parametrize("B,N,H,T", [(3, 7, 16, 1), (7, 64, 32, 1), (6, 33, 64, 0), (70, 18, 32, 1), (6, 130, 16, 0)])
+def test_compact_output_is_zero_where_no_pair_lies(B, N, H, T, monkeypatch):
+    """coupling_bias in the compacted layout into memory that holds NaN: the pairs of the plain layout
+    (bit for bit) and zeros everywhere else - row pads of every length, tails, walkers with no, one
+    and every site."""
     from hamiltonzero_amd import kernels, pair_bias
 
     print(f"[case] compact zeros B={B} N={N} H={H} T={T}", flush=True)
@@ -278,11 +279,51 @@ def test_compact_output_is_zero_where_no_pair_lies(B, N, H, T):
     mask[0] = False
     mask[1] = False
     mask[1, N // 2] = True
+    if B >= 6:  # counts of every remainder of 4 (row pads of 0 to 3), and the largest
+        for b, n in enumerate((N, N - N % 4 - 4, N - N % 4 - 3, N - N % 4 - 2, N - N % 4 - 1)[: B - 2], start=2):
+            mask[b] = torch.randperm(N, generator=gen, device="cuda") < n
     edge, edge_t = rnd(B, N, N, C), (rnd(B, N, N, C) if T else None)
     opts = dict(d_head=16, inner_gain=0.5, mask=mask, edge_t=edge_t)
     plain = pair_bias.coupling_bias(edge, params, **opts)
-    dirty = [torch.full(kernels.e_shape(B, N, H, "compact"), float("nan"), device="cuda") for _ in range(1 + T)]
-    del dirty  # the caching allocator hands this memory out again
+    monkeypatch.setattr(torch, "empty", lambda shape, **kw: torch.full(shape, float("nan"), **kw))
     got = pair_bias.coupling_bias(edge, params, e_layout="compact", **opts)
+    monkeypatch.undo()
     for a, b in zip(got if T else (got,), plain if T else (plain,)):
         assert torch.equal(a, kernels.compact_bias(b, mask))
+
+
+@pytest.mark.parametrize("kind", ["trunk", "tree"])
+def test_producers_with_edges_at_the_end_of_float32(kind):
+    """One pair's edge with a value above the largest bfloat16, one with an infinity, one with a NaN.
+    In float32 the first has a mean square of infinity, so its normalised values are zeros: the trunk
+    gives what it gives for an edge of zeros (its norm comes first), the tree b_out / 4. The others'
+    results are NaN, and every other pair, those of the same tile of 16 or 32 among them, is bit for
+    bit what it is without them."""
+    from hamiltonzero_amd import pair_bias
+
+    print(f"[case] extreme edges {kind}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    rnd = lambda *s: torch.randn(s, generator=gen, device="cuda")  # noqa: E731
+    B, N, C, H = 2, 9, 96, 16
+    hid = 64 if kind == "trunk" else 128
+    p = {"w_in": rnd(C, hid) / 10, "b_in": rnd(hid), "w_out": rnd(hid, H) / 8, "b_out": rnd(H)}
+    if kind == "trunk":
+        p.update(ln_w=1 + 0.1 * rnd(C), w_1=rnd(hid, hid) / 8, b_1=rnd(hid), w_2=rnd(hid, hid) / 8, b_2=rnd(hid))
+        call = lambda x: pair_bias.coupling_bias(x, p, d_head=16, inner_gain=0.5)  # noqa: E731
+    else:
+        p.update(norm_w=1 + 0.1 * rnd(1, hid), w_1=rnd(1, hid, hid) / 11, b_1=rnd(1, hid),
+                 w_2=rnd(1, hid, hid) / 11, b_2=rnd(1, hid), out_norm_w=1 + 0.1 * rnd(hid))
+        call = lambda x: pair_bias.mlp_bias(x, p, d_head=16, e_layout="qhk")  # noqa: E731
+    edge = rnd(B, N, N, C)
+    plain = call(edge)  # [B, N, H, N]
+    for c, value in enumerate((3.4e38, float("inf"), float("nan"))):
+        edge[0, 1, 2 + c] = 0.0
+    zeros = call(edge)[0, 1, :, 2]
+    for c, value in enumerate((3.4e38, float("inf"), float("nan"))):
+        edge[0, 1, 2 + c, 5] = value
+    got = call(edge)
+    want = zeros if kind == "trunk" else p["b_out"] / 4
+    assert torch.all((got[0, 1, :, 2] - want).abs() <= TOL * want.abs().max())
+    assert torch.isnan(got[0, 1, :, 3:5]).all()
+    got[0, 1, :, 2:5] = plain[0, 1, :, 2:5]
+    assert torch.equal(got, plain)

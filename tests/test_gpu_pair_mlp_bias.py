@@ -126,6 +126,23 @@ def test_pair_mlp_bias_hidden_128_rounds(B, N, C, H, T, mask_kind, layout):
                                        layout))
 
 
+@pytest.mark.parametrize(
+    "B,Nq,Nk,H,T,extra,row_offset,mask_kind,layout",
+    [
+        (3, 20, 20, 16, 1, False, 0, "key", "qkh"),          # keys listed, every query row
+        (4, 17, 17, 16, 0, False, 0, "key_empty", "qhk"),    # a walker without a key takes every pair
+        (2, 9, 70, 32, 1, False, 40, "key_empty", "qkh"),    # a list over two ballots, a row offset
+        (2, 33, 12, 16, 1, True, 7, "key", "qhk"),           # the extra channel and its tangent
+        (3, 14, 14, 32, 0, True, 0, "square_empty", "qkh"),  # the extra channel without one
+    ],
+)
+def test_pair_mlp_bias_hidden_128_lists_and_extra(B, Nq, Nk, H, T, extra, row_offset, mask_kind, layout):
+    """Hidden width 128 and 96 channels (the kernel whose weights pass through the LDS): the key
+    mask's lists and the extra input channel."""
+    test_pair_mlp_bias_matches_oracle((f"lists_{B}_{Nq}_{Nk}_{H}", B, Nq, Nk, 96, 128, H, 1, T, extra, True,
+                                       row_offset, mask_kind, layout))
+
+
 def test_pair_mlp_bias_feeds_the_gated_rect_attention():
     """The large-N chain (sequence_trunk.py:962-984): the producer's bias with a global row
     offset, then the gated rectangular attention, against the oracle's chain."""
