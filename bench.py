@@ -53,6 +53,8 @@ TREE_BIAS_METRIC = ("tree coupling-bias producer (normalised pair MLP + LCA-ALiB
 HBM_PEAK_GBS = 8000.0
 FP32_PEAK_TFLOPS = 157.3
 BF16_PEAK_TFLOPS = 2516.6
+# float32 products formed as six bfloat16 ones (csrc/split_f32.h): the bias producers, the executor
+F32X6_PEAK_TFLOPS = BF16_PEAK_TFLOPS / 6
 INFINITY_CACHE_BYTES = 256 << 20
 
 
@@ -270,7 +272,8 @@ def rect_algorithmic(B, Nq, Nk, H, D, n_phys):
 
 
 def roofline(bytes_, flops, t_s, dtype):
-    peak_c = BF16_PEAK_TFLOPS if dtype == "bf16" else FP32_PEAK_TFLOPS
+    """``dtype``: "bf16", "f32" (the float32 matrix instruction) or "f32x6"."""
+    peak_c = {"bf16": BF16_PEAK_TFLOPS, "f32": FP32_PEAK_TFLOPS, "f32x6": F32X6_PEAK_TFLOPS}[dtype]
     t_hbm = bytes_ / (HBM_PEAK_GBS * 1e9)
     t_cmp = flops / (peak_c * 1e12)
     if t_hbm >= t_cmp:
@@ -278,6 +281,20 @@ def roofline(bytes_, flops, t_s, dtype):
         return {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS}
     ach = flops / t_s / 1e12
     return {"bound": "mfma", "achieved": ach, "peak": peak_c, "unit": "TFLOP/s", "frac": ach / peak_c}
+
+
+def wavefn_flops(B, n, d_q, d_z, R_leaf, G, d_r, R_merge, R_out):
+    """A leaf is linear and a first-level node bilinear in a site's d_q inputs: their products are
+    needed on as many rows as those inputs have directions, where that is fewer than the walkers."""
+    dm = G * d_r
+    node = 2 * G * d_r ** 3 + 4 * dm * R_merge
+    flops = 2 * n * min(B, d_q) * (d_z * R_leaf + R_leaf * dm) + 2 * B * (dm * R_out + R_out * 2)
+    if n > 1:
+        pairs = n // 2
+        flops += pairs * min(B, d_q * d_q) * node + B * (n - 1 - pairs) * node
+        if B > d_q * d_q:
+            flops += pairs * 2 * B * d_q * d_q * dm
+    return flops
 
 
 def traffic_from_profile(config):
@@ -748,8 +765,8 @@ def run_pair_mlp(args, cfg):
     pairs = B * n_phys * n_phys
     flops_pair = 2 * 2 * (C * Hd + 2 * nb * Hd * Hd + Hd * H)  # primal and tangent
     bytes_pair = 4 * (2 * C + 2 * H)
-    roof = roofline(pairs * bytes_pair, pairs * flops_pair, t_s, "f32")
-    roof.update({"kernel": "pair_mlp_bias_kernel", "traffic": traffic_from_profile(args.config),
+    roof = roofline(pairs * bytes_pair, pairs * flops_pair, t_s, "f32x6")
+    roof.update({"kernel": "pair_mlp_bias_wide_kernel", "traffic": traffic_from_profile(args.config),
                  "basis": f"computed pairs ({pairs}: the {n_phys} x {n_phys} physical pairs of each walker) x "
                           f"{flops_pair} flops / {bytes_pair} bytes (edge, edge_t in; e, e_t out)",
                  "bytes_per_step": pairs * bytes_pair, "flops_per_step": pairs * flops_pair,
@@ -829,7 +846,7 @@ def run_executor(args, cfg):
     # The dominant kernel, the merge, timed on its own over the same number of launches.
     ms_merge = timed(merge, args.steps, args.warmup, stream)
     ms_apply = timed(apply, args.steps, args.warmup, stream)
-    roof = roofline(4 * (3 * M * dm + G * R ** 3), merge_flops, ms_merge / 1e3, "f32")
+    roof = roofline(4 * (3 * M * dm + G * R ** 3), merge_flops, ms_merge / 1e3, "f32x6")
     roof["traffic"] = traffic_from_profile(args.config)
     roof["kernel"] = "hz::quadrilinear_merge_kernel"
     roof["basis"] = ("algorithmic flops of the merge launch, 2 M G d_r^3 (d_r outputs per group, each a "
@@ -941,7 +958,7 @@ def run_trunk(args, cfg):
     fl_pair = 2 * (C * HID + 2 * HID * HID + HID * H)
     flops_eff, flops_all = 2 * fl_pair * pairs_eff, 2 * fl_pair * pairs_all
     bytes_eff = pairs_eff * 4 * (2 * C + 2 * H)
-    roof = roofline(bytes_eff, flops_eff, ms_prod / 1e3, "f32")
+    roof = roofline(bytes_eff, flops_eff, ms_prod / 1e3, "f32x6")
     roof["traffic"] = traffic_from_profile(args.config)
     roof["kernel"] = "hz::pair_bias_kernel<96,2,true>"
     roof["basis"] = ("the producer launch: 2 x (C d_h + 2 d_h^2 + d_h H) x 2 flops per computed pair (primal and "
@@ -1028,15 +1045,13 @@ def run_wavefn(args, cfg):
 
     ms = timed(step, args.steps, args.warmup, stream)
     rows = B * n
-    merge_rows = B * (n - 1)  # every level's nodes: n/2 + n/4 + ... + 1 per walker
-    flops = (2 * rows * (d_q * d_z + d_z * R_leaf + R_leaf * dm)
-             + merge_rows * (2 * G * d_r ** 3 + 2 * (dm * R_merge + R_merge * dm))
-             + 2 * B * (dm * R_out + R_out * 2))
-    roof = roofline(4 * (rows * d_q + B * 2), flops, ms / 1e3, "f32")
+    flops = wavefn_flops(B, n, d_q, d_z, R_leaf, G, d_r, R_merge, R_out)
+    roof = roofline(4 * (rows * d_q + B * 2), flops, ms / 1e3, "f32x6")
     roof["traffic"] = traffic_from_profile(args.config)
     roof["kernel"] = "hz_compiled_wavefunction (every launch of the step)"
-    roof["basis"] = ("algorithmic flops of the step: the leaf GEMMs 2 B n (d_q d_z + d_z R_leaf + R_leaf d_m), per "
-                     "merged node 2 G d_r^3 + 4 d_m R_merge, the readout; per average step duration")
+    roof["basis"] = ("flops the step cannot do without: the leaf on min(B, d_q) rows a site, the first level on "
+                     "min(B, d_q^2) rows a pair and the walkers' sums over them, per later node of a walker 2 G d_r^3 "
+                     "+ 4 d_m R_merge, the readout; per average step duration")
     roof["flops_per_step"] = flops
     cpu = None
     if not args.no_cpu_baseline:

@@ -57,6 +57,21 @@ def test_multi_gpu_request_is_refused():
     assert "one GPU" in r.stderr
 
 
+def test_wavefunction_flops():
+    """Every walker's rows where the walkers are few; a basis of the inputs' directions where not."""
+    node, leaf, out = 2 * 48 * 32 ** 3 + 4 * 1536 * 1024, 2 * (32 * 1536 + 1536 * 1536), 2 * (1536 * 64 + 128)
+    few = bench.wavefn_flops(3, 8, 4, 32, 1536, 48, 32, 1024, 64)
+    assert few == 3 * (8 * leaf + 7 * node + out)
+    many = bench.wavefn_flops(1024, 64, 4, 32, 1536, 48, 32, 1024, 64)
+    assert many == 64 * 4 * leaf + 32 * 16 * node + 32 * 1024 * 2 * 16 * 1536 + 1024 * (31 * node + out)
+    assert bench.wavefn_flops(5, 1, 4, 32, 64, 3, 32, 32, 16) == 4 * 2 * (32 * 64 + 64 * 96) + 5 * 2 * (96 * 16 + 32)
+
+
+def test_products_of_six_are_priced_at_a_sixth_of_the_bf16_peak():
+    r = bench.roofline(1.0, 1e12, 1.0, "f32x6")
+    assert r["bound"] == "mfma" and r["peak"] == pytest.approx(2516.6 / 6)
+
+
 def test_merge_level_config_is_fine_tune_shaped():
     """The executor bench leg runs one tree level at the fine-tune ranks (config.py:21-29):
     48 groups of d_r = 32 (merge_dim 1536), merge_rank 1024, 1024 walkers x 32 node pairs."""
