@@ -856,7 +856,7 @@ __global__ void __launch_bounds__(256) leaf_basis_kernel(const float* __restrict
 // owns 16 rows x 32 columns, its four waves every fourth K block of 16 each, summed through LDS in
 // order. v_mfma_f64_16x16x4_f64, lane l = 16 g + c: A[row c][k g], B[k g][col c], C/D element r at
 // [row g + 4 r][col c]; a lane's four k of a block are 4 g .. 4 g + 3 in both operands, its two columns
-// neighbours. N is a multiple of 32. 39 us for 256 x 1536 x 1536 (15 at the 64-bit matrix rate): few
+// neighbours. N is a multiple of 32. 34 us for 256 x 1536 x 1536 (15 at the 64-bit matrix rate): few
 // workgroups, each waiting for its operands.
 __global__ void __launch_bounds__(256) basis_gemm_f64_kernel(const double* __restrict__ A, const float* __restrict__ Bm,
                                                              double* __restrict__ C, int64_t M, int N, int K) {
@@ -873,26 +873,30 @@ __global__ void __launch_bounds__(256) basis_gemm_f64_kernel(const double* __res
     acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, static_cast<double>(b1), acc[1], 0, 0, 0);
   };
   const int whole = K / 16;
-  // a block's operands, loaded under the products of the one before
-  double a[4], an[4];
-  float2 b[4], bn[4];
-  auto load = [&](int t, double (&a)[4], float2 (&b)[4]) {
-    const int k0 = 16 * t + 4 * g;
+  // this wave's blocks wave, wave + 4, ..., the operands of three in flight beside one's products
+  constexpr int kDeep = 4;
+  const int mine = (whole - wave + 3) >> 2;
+  double a[kDeep][4];
+  float2 b[kDeep][4];
+  auto load = [&](int i, double (&a)[4], float2 (&b)[4]) {
+    const int k0 = 16 * (wave + 4 * (i < mine ? i : mine - 1)) + 4 * g;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       a[j] = ar[k0 + j];
       b[j] = *reinterpret_cast<const float2*>(bc + static_cast<int64_t>(k0 + j) * N);
     }
   };
-  if (wave < whole) load(wave, a, b);
-  for (int t = wave; t < whole; t += 4) {
-    load(t + 4 < whole ? t + 4 : t, an, bn);
+  if (mine > 0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) step(a[j], b[j].x, b[j].y);
+    for (int i = 0; i < kDeep - 1; ++i) load(i, a[i], b[i]);
+    for (int i0 = 0; i0 < mine; i0 += kDeep) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      a[j] = an[j];
-      b[j] = bn[j];
+      for (int i = 0; i < kDeep; ++i) {
+        if (i0 + i == mine) break;
+        load(i0 + i + kDeep - 1, a[(i + kDeep - 1) % kDeep], b[(i + kDeep - 1) % kDeep]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) step(a[i][j], b[i][j].x, b[i][j].y);
+      }
     }
   }
   if (whole * 16 < K && wave == (whole & 3)) {  // the last K block, zeros past K
@@ -1113,7 +1117,7 @@ __global__ void __launch_bounds__(256) leaf_pair_level_kernel(const float* __res
 // that fit its one K step, and no more basis rows than walker rows, neither at the leaves (2 nq: the
 // basis in 64 bits and its factors take half a leaf buffer each as floats) nor at the pairs (nq^2);
 // R in 64 bits fits where z is not needed. At that line (nq = 4, fine-tune widths) the whole
-// wavefunction takes 319 us for 16 walkers of 8 sites with it and 436 for 15 without, 532 and 657
+// wavefunction takes 312 us for 16 walkers of 8 sites with it and 433 for 15 without, 522 and 653
 // at 64 sites.
 bool basis_serves(int64_t B, int n, int nq, int d_z) {
   const int64_t nq2 = static_cast<int64_t>(nq) * nq;
