@@ -8,8 +8,8 @@
 // so b is split once and stays in registers, T_i streams through LDS in chunks of four k (48 KB
 // for two chunks), split as it is staged, and the outer sum is one multiply-add per element of
 // w_k in the matrix cores' output layout (16 vector instructions per 12 matrix ones). Bound by the
-// matrix cores' power: 73% busy at 1.66 GHz, 209 TFLOP/s of float32 products at 16384 rows, G = 48
-// (246 us; 514 with the contraction over (k, l) on the float32 matrix instruction).
+// matrix cores' power: 72% busy at 1.65 GHz, 206 TFLOP/s of float32 products at 32768 rows, G = 48
+// (500 us; 1018 with the contraction over (k, l) on the float32 matrix instruction).
 //
 // Factorized apply: two launches of one tiled GEMM, C = A B with A [M, K], B [K, N]
 // row-major; the first multiplies its result by the conditioner row of each output row

@@ -29,9 +29,9 @@
 // waves: two a SIMD, so one wave's splits and activations run under the other's products. A tile's
 // 384 matrix instructions take 6144 cycles beside about 1400 vector instructions (5600 cycles);
 // with two waves a SIMD they overlap by a third. 1024 walkers of 36 sites, C = 96, 32 heads, with
-// tangent: 495 us (760 on the float32 matrix instruction); 250 us of that with neither the products
-// nor memory, 90 us for the products beyond it, 95 us for the loads and stores. Twelve waves spill
-// and take 545 us.
+// tangent: 520 us (751 on the float32 matrix instruction), 572 where it zeroes the compacted layout's
+// unfilled entries too. Of 495 us in one session: 250 with neither the products nor memory, 90 for
+// the products beyond it, 95 for the loads and stores. Twelve waves spill and take 545 us.
 //
 // A tile is 16 pairs with their tangent (T = 1: N block 0 primal, N block 1 tangent) or 32
 // pairs (T = 0). With a mask, only pairs whose key site is physical are computed (and, in

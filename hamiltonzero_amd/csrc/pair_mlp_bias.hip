@@ -438,8 +438,8 @@ __global__ void __launch_bounds__((64 * PMShape<C, KB, HB>::NW), (KB == 8 ? 1 : 
 // eight waves (two a SIMD) each run their own tile of 16 pairs with tangent (32 without) in step,
 // so a staged step serves eight tiles; a workgroup's rounds cover an item's tiles eight at a time
 // and waves past its end only stage. 1024 walkers of 36 sites, C = 96, 16
-// heads, with tangent: 1310 us (2290 on the float32 matrix instruction), matrix cores 54% busy at
-// 1.92 GHz; what is left is the vector work of the splits and the wait for each round's rows.
+// heads, with tangent: 1310 us (2275 on the float32 matrix instruction), matrix cores 49% busy at
+// 2.25 GHz; what is left is the vector work of the splits and the wait for each round's rows.
 template <int C, int HB>
 struct PWShape {
   static constexpr int KB = 8, HID = 128, H = 16 * HB, NW = 8, NT = 64 * NW;

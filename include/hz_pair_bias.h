@@ -27,6 +27,8 @@
  * 1 <= N <= HZ_MAX_N, B >= 1, T in {0, 1}. inner_gain = n_layers^-1/2 (trunk.py:61),
  * eps = 1e-5 (odd_ops.py:185), bias_div = sqrt(d_head) (trunk.py:103-105).
  *
+ * Finite edges give what float32 arithmetic gives; a weight or a hidden value that is not finite, or
+ * above the largest bfloat16 (3.39e38), may give NaN where float32 gives an infinity.
  * HZ_FLAG_E_ZERO (with HZ_FLAG_E_COMPACT): the rest of every block is written as zeros, so e and e_t
  * may be uninitialised memory. Without it, what no pair fills is left untouched.
  * HZ_FLAG_E_COMPACT (hz_mhsea.h): e / e_t in the compacted physical-pair layout [B, H, N,
