@@ -370,6 +370,54 @@ def test_pair_basis_of_inputs_that_cancel(rows):
     assert np.all(dphi <= TOL * np.pi + 1e-6 * kappa), (dphi.max(), kappa[np.argmax(dphi)])
 
 
+@pytest.mark.parametrize(
+    "B,n,d_q,d_z,R_leaf,G",
+    [
+        (32, 4, 4, 1, 37, 2),    # R fills z to the last float; every leaf's basis has one row
+        (31, 4, 4, 1, 37, 2),    # one walker fewer: it does not fit, the plain path
+        (2, 2, 1, 1, 1, 1),      # the smallest of everything
+        (18, 2, 3, 2, 15, 64),   # less than one K block; the widest carrier (2048); two rows of three
+        (20, 16, 2, 3, 130, 33), # eight K blocks and a remainder, a row of 16 that is not full
+        (17, 8, 4, 9, 80, 5),    # five whole K blocks: one wave has two
+    ],
+)
+def test_pair_basis_sizes(B, n, d_q, d_z, R_leaf, G):
+    """The leaf basis in 64 bits: contraction lengths either side of its blocks, column and row counts
+    either side of its tiles, fewer independent rows than inputs, the workspace's exact fit."""
+    from hamiltonzero_amd import executor
+
+    _say(f"wavefunction basis sizes B={B} n={n} d_q={d_q} d_z={d_z} R_leaf={R_leaf} G={G}")
+    p = _wavefn_case(B + n + R_leaf, B, n, d_q, d_z, R_leaf, G, 36, 12, "random")
+    kernel, tree, q = _namespaces(p)
+    la, ph = executor.execute_wavefunction(kernel, tree, q)
+    torch.cuda.synchronize()
+    want_la, want_ph = X.execute_wavefunction(**p)
+    kappa = _readout_condition(p)
+    dla = np.abs(la.cpu().numpy().astype(np.float64) - want_la)
+    assert np.all(dla <= TOL * np.max(np.abs(want_la)) + 1e-6 * kappa), (dla.max(), kappa[np.argmax(dla)])
+    dphi = np.abs(np.angle(np.exp(1j * (ph.cpu().numpy().astype(np.float64) - want_ph))))
+    assert np.all(dphi <= TOL * np.pi + 1e-6 * kappa), (dphi.max(), kappa[np.argmax(dphi)])
+
+
+@pytest.mark.parametrize("where", ["q", "leaf_U", "leaf_h"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_pair_basis_of_values_that_are_not_finite(where, value):
+    """What is not finite stays so, and only where it belongs: one walker's input, or a weight (every
+    walker) or one leaf's conditioner (every walker whose tree holds that leaf)."""
+    from hamiltonzero_amd import executor
+
+    _say(f"wavefunction basis, {value} in {where}")
+    p = _wavefn_case(3, 20, 4, 4, 20, 40, 2, 36, 12, "all")
+    kernel, tree, q = _namespaces(p)
+    clean = [x.cpu().numpy() for x in executor.execute_wavefunction(kernel, tree, q)]
+    p[where].reshape(-1)[(7 * 4 + 1) * 4 + 2 if where == "q" else 11] = value  # q: walker 7, site 1
+    kernel, tree, q = _namespaces(p)
+    got = [x.cpu().numpy() for x in executor.execute_wavefunction(kernel, tree, q)]
+    hit = np.arange(20) == 7 if where == "q" else np.ones(20, bool)
+    for a, b in zip(got, clean):
+        assert np.all(np.isnan(a[hit])) and np.array_equal(a[~hit], b[~hit])
+
+
 def test_compiled_wavefunction_structure_errors():
     from hamiltonzero_amd import executor
 
