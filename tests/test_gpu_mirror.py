@@ -150,3 +150,45 @@ def test_op_level_edge_attention(n, d, batched):
     assert rel(got, want) <= TOL
     assert rel(got_ref, want_ref) <= TOL
     assert rel(got_ref[0].cpu().numpy(), O.reference_edge_attention(Q[0], K[0], V[0], E[0], M[0])) <= TOL
+
+
+@pytest.mark.parametrize("given", [("q",), ("k", "v"), ("e",)])
+@pytest.mark.parametrize("N,D,layout", [(16, 8, "qhk"), (64, 32, "qhk"), (64, 16, "qkh"), (45, 32, "qkh"), (64, 16, "compact"),
+                                        (64, 64, "qhk"), (130, 32, "qhk"), (96, 64, "qkh")])
+def test_forward_mode_of_some_operands(N, D, layout, given):
+    """Operands without a tangent reach the kernels as none: the same as tangents of zeros, in every
+    kernel family and bias layout (float32 sums of the same terms, 1e-5 of the largest)."""
+    import torch.autograd.forward_ad as fwAD
+
+    from hamiltonzero_amd import kernels, mhsea_tuned
+
+    print(f"[case] some tangents N={N} D={D} {layout} {given}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(N + D)
+    rnd = lambda *s: torch.randn(s, generator=gen, device="cuda")  # noqa: E731
+    B, H = 3, 4
+    x = {n: rnd(B, N, H, D) * D ** -0.5 for n in "qkv"}
+    mask = torch.rand((B, N), generator=gen, device="cuda") < 0.7
+    t = {n: rnd(B, N, H, D) for n in "qkv"}
+    if layout == "compact":
+        x["e"], t["e"] = (kernels.compact_bias(rnd(B, N, H, N), mask) for _ in range(2))
+    else:
+        x["e"], t["e"] = rnd(*kernels.e_shape(B, N, H, layout)), rnd(*kernels.e_shape(B, N, H, layout))
+    full = {n: t[n] if n in given else torch.zeros_like(t[n]) for n in "qkve"}
+    out, lse = kernels.mhsea_fwd(x["q"], x["k"], x["v"], mask, x["e"], e_layout=layout)
+    want = kernels.mhsea_jvp(x["q"], x["k"], x["v"], mask, out, lse, full["q"], full["k"], full["v"], x["e"], full["e"],
+                             e_layout=layout)
+    with fwAD.dual_level():
+        duals = {n: fwAD.make_dual(x[n], t[n]) if n in given else x[n] for n in "qkve"}
+        y, _ = mhsea_tuned.mhsea_ad(duals["q"], duals["k"], duals["e"], duals["v"], mask, e_layout=layout)
+        got = fwAD.unpack_dual(y).tangent
+    assert torch.all((got - want).abs() <= 1e-5 * want.abs().max())
+    if layout == "compact":
+        return
+    _, want = kernels.mhsea_fwd_jvp_gated(x["q"], x["k"], x["v"], mask, full["q"], full["k"], full["v"], e=x["e"],
+                                          et=full["e"], e_layout=layout)
+    with fwAD.dual_level():  # where a gradient is wanted beside the tangent
+        duals = {n: x[n].clone().requires_grad_() for n in "qkve"}
+        duals = {n: fwAD.make_dual(v, t[n]) if n in given else v for n, v in duals.items()}
+        y = mhsea_tuned.gated_edge_attention(duals["q"], duals["k"], duals["e"], duals["v"], mask, e_layout=layout)
+        got = fwAD.unpack_dual(y).tangent
+    assert torch.all((got - want).abs() <= 1e-5 * want.abs().max())
